@@ -118,54 +118,24 @@ BTRC_HD uint32_t permutation_element_masked(uint32_t i, uint32_t l, uint32_t w, 
     return mod_recip(i + p, l, m);
 }
 
-BTRC_HD uint32_t permutation_element(uint32_t i, uint32_t l, uint32_t p)
+// Quotient and remainder of a by a small base with m = floor((2^32 - 1) /
+// base): mulhi(a, m) > a / base - 1, so one correction step gives the exact
+// quotient.
+BTRC_HD void divmod_recip(uint32_t a, uint32_t base, uint32_t m, uint32_t *q, uint32_t *r)
 {
-    return permutation_element_masked(i, l, permutation_mask(l), 0xffffffffu / l, p);
-}
-
-// Quotient and remainder of a by a small base; a stays below 2^32 for every
-// image this tracer renders, which keeps the division in 32 bits. There it
-// multiplies by m = floor((2^32 - 1) / base): mulhi(a, m) > a / base - 1, so
-// one correction step gives the exact quotient.
-BTRC_HD void divmod_base(uint64_t a, uint32_t base, uint32_t m, uint64_t *q, uint64_t *r)
-{
-    if(a < 0x100000000ull)
+    uint32_t q32 = mulhi32(a, m);
+    uint32_t r32 = a - q32 * base;
+    if(r32 >= base)
     {
-        const uint32_t a32 = (uint32_t)a;
-        uint32_t q32 = mulhi32(a32, m);
-        uint32_t r32 = a32 - q32 * base;
-        if(r32 >= base)
-        {
-            q32 = q32 + 1;
-            r32 = r32 - base;
-        }
-        *q = q32;
-        *r = r32;
+        q32 = q32 + 1;
+        r32 = r32 - base;
     }
-    else
-    {
-        const uint64_t q64 = a / base;
-        *q = q64;
-        *r = a - q64 * base;
-    }
+    *q = q32;
+    *r = r32;
 }
 
-// One digit of owen_scrambled_radical_inverse (low_discrepancy.cpp:83-101):
-// the lowest base-`base` digit of a, permuted by the hash of the digits
-// reversed so far, appended to them; a loses the digit. m and w are the
-// base's reciprocal (divmod_base) and permutation mask.
-BTRC_HD uint64_t owen_digit(uint32_t base, uint32_t m, uint32_t w, uint64_t hash, uint64_t &a, uint64_t reversed)
-{
-    uint64_t next, digit_value;
-    divmod_base(a, base, m, &next, &digit_value);
-    const uint64_t digit_hash = mix_bits(hash ^ reversed);
-    digit_value = permutation_element_masked((uint32_t)digit_value, base, w, m, (uint32_t)digit_hash);
-    a = next;
-    return reversed * base + digit_value;
-}
-
-// owen_scrambled_radical_inverse, low_discrepancy.cpp:83-101 (the digit
-// split's reciprocal and the permutation's mask computed once per call)
+// owen_scrambled_radical_inverse, low_discrepancy.cpp:83-101, for any a. The
+// tracer's stages use halton_value below (a < 2^32, the same numbers).
 BTRC_HD float owen_scrambled_radical_inverse(uint32_t base, uint64_t a, uint64_t hash)
 {
     const float inv_base = 1.0f / (float)base;
@@ -175,72 +145,193 @@ BTRC_HD float owen_scrambled_radical_inverse(uint32_t base, uint64_t a, uint64_t
     uint64_t reversed_digits = 0;
     while(1.0f - inv_base_m < 1.0f)
     {
-        uint64_t next, digit_value;
-        divmod_base(a, base, m, &next, &digit_value);
-        const uint64_t digit_hash = mix_bits(hash ^ reversed_digits);
-        digit_value = permutation_element_masked((uint32_t)digit_value, base, w, m, (uint32_t)digit_hash);
-        reversed_digits = reversed_digits * base + digit_value;
+        const uint64_t next = a / base;
+        const uint32_t digit = (uint32_t)(a - next * base);
+        const uint32_t digit_hash = (uint32_t)mix_bits(hash ^ reversed_digits);
+        reversed_digits = reversed_digits * base + permutation_element_masked(digit, base, w, m, digit_hash);
         inv_base_m = inv_base_m * inv_base;
         a = next;
     }
     return fmin_(inv_base_m * (float)reversed_digits, 0x1.fffffep-1f);
 }
 
-// Tables of the first digits. The first K scrambled digits of a depend only
-// on a mod base^K, so for the first HALTON_TABLE_DIMS dimensions a table
-// holds, for every r < base^K (K the largest with base^K <= 4096), the
-// reversed digits after K steps of the loop above on a = r. The rest of the
-// digits continue the loop from there; results are identical.
-constexpr int HALTON_TABLE_DIMS = 256;
-constexpr uint32_t HALTON_TABLE_SPAN = 4096;
-
-// a dimension's table: where its values start, base^K, K, and
-// floor((2^32 - 1) / base^K) for divmod_base
-struct HaltonDim
+// A dimension of the sampler as the tracer's stages read it (two 16-byte
+// loads): the constants of its digit loop, and its first-digit table. The
+// first K scrambled digits of a depend only on a mod base^K, so a table of
+// base^K reversed K-digit strings (HALTON_TABLE_SPAN bounds base^K) replaces
+// K steps of the loop; the rest of the digits continue from there.
+struct alignas(16) HaltonDim
 {
-    uint32_t first, span, digits, recip;
+    uint32_t base;          // the dimension's prime | digits after the table << 16 | K << 20 | bits of its permutation << 28
+    uint32_t recip;         // floor((2^32 - 1) / prime)
+    uint32_t hash_lo, hash_hi; // mix_bits(1 + (dim << 4))
+    uint32_t first;         // the table's first value
+    uint32_t span;          // base^K
+    uint32_t span_recip;    // floor((2^32 - 1) / span)
+    float scale;            // 1 / base^digits, rounded as the digit loop rounds it
 };
+
+// Up to 2^16 entries per dimension: K = 6 for base 5, 4 for 13, 3 to 37, 2 to
+// 251, 1 beyond; 5.0 million 16-bit values in all, most of a path's
+// dimensions in the first megabytes.
+constexpr uint32_t HALTON_TABLE_SPAN = 65536;
 
 struct HaltonTables
 {
     const uint16_t *values; // all dimensions' tables
-    const HaltonDim *dims;  // HALTON_TABLE_DIMS entries
+    const HaltonDim *dims;  // PRIME_TABLE_SIZE entries
 };
 
-// the same as owen_scrambled_radical_inverse(base, a, hash) with the first
-// info.digits digits from table t
-BTRC_HD float owen_scrambled_radical_inverse_tabled(uint32_t base, uint64_t a, uint64_t hash, const uint16_t *t,
-                                                    HaltonDim info)
+// one dimension's record; its table starts at `first`
+BTRC_HD HaltonDim halton_dim(uint32_t base, uint32_t dim, uint32_t first)
 {
-    const float inv_base = 1.0f / (float)base;
-    const uint32_t m = 0xffffffffu / base;
-    const uint32_t w = permutation_mask(base);
-    uint64_t high, low;
-    divmod_base(a, info.span, info.recip, &high, &low); // a / base^K, a mod base^K
-    uint64_t reversed_digits = t[info.first + low];
-    a = high;
-    float inv_base_m = 1.0f;
-    for(uint32_t k = 0; k < info.digits; ++k)
-        inv_base_m = inv_base_m * inv_base;
-    while(1.0f - inv_base_m < 1.0f)
+    HaltonDim d;
+    uint32_t span = 1, k = 0, digits = 0, bits = 0;
+    while((uint64_t)span * base <= HALTON_TABLE_SPAN)
     {
-        reversed_digits = owen_digit(base, m, w, hash, a, reversed_digits);
-        inv_base_m = inv_base_m * inv_base;
+        span *= base;
+        ++k;
     }
-    return fmin_(inv_base_m * (float)reversed_digits, 0x1.fffffep-1f);
+    const float inv_base = 1.0f / (float)base;
+    d.scale = 1.0f;
+    for(; 1.0f - d.scale < 1.0f; ++digits)
+        d.scale = d.scale * inv_base;
+    while((permutation_mask(base) >> bits) != 0)
+        ++bits;
+    const uint64_t hash = mix_bits((uint64_t)(1u + (dim << 4)));
+    d.base = base | ((digits - k) << 16) | (k << 20) | (bits << 28);
+    d.recip = 0xffffffffu / base;
+    d.hash_lo = (uint32_t)hash;
+    d.hash_hi = (uint32_t)(hash >> 32);
+    d.first = first;
+    d.span = span;
+    d.span_recip = 0xffffffffu / span;
+    return d;
 }
 
-// inverse_radical_inverse, low_discrepancy.cpp:103-114
-BTRC_HD uint64_t inverse_radical_inverse(uint64_t inverse, uint32_t base, int digits)
+// product modulo 2^24 (its upper bits are arbitrary): 24-bit multiplies issue
+// at the full rate on gfx950, 32-bit ones at a quarter of it
+BTRC_HD uint32_t mul24(uint32_t a, uint32_t b)
 {
-    uint64_t index = 0;
-    for(int i = 0; i < digits; ++i)
+#ifdef __HIP_DEVICE_COMPILE__
+    return __umul24(a, b);
+#else
+    return (a & 0xffffffu) * (b & 0xffffffu);
+#endif
+}
+
+// bits [at, at + n) of x, n >= 0 and below 32
+BTRC_HD uint32_t bit_field(uint32_t x, uint32_t at, uint32_t n)
+{
+#ifdef __HIP_DEVICE_COMPILE__
+    return __builtin_amdgcn_ubfe(x, at, n);
+#else
+    return (x >> at) & ((1u << n) - 1u);
+#endif
+}
+
+// Digits of the scrambled radical inverse after the first ones: `n` lowest
+// digits of a, each permuted by the hash of the digits reversed so far and
+// appended to `reversed` (below 2^32 before every step: the loop ends once
+// base^digits reaches 2^25). Kensler's permutation as in
+// permutation_element_masked, restricted to what its result depends on: the
+// right shifts take bits below `bits` only (the base's width, at most 13), so
+// every product is needed modulo 2^bits alone and 24-bit multiplies do. Seven
+// quarter-rate products a digit become full-rate ones.
+BTRC_HD uint64_t halton_digits(const HaltonDim &d, uint32_t n, uint32_t a, uint32_t reversed)
+{
+    const uint32_t base = d.base & 0xffffu, bits = d.base >> 28;
+    const uint32_t b1 = bits - 1, b2 = bits > 2 ? bits - 2 : 0, b4 = bits > 4 ? bits - 4 : 0,
+                   b11 = bits > 11 ? bits - 11 : 0;
+    const uint64_t hash = (uint64_t)d.hash_lo | ((uint64_t)d.hash_hi << 32);
+    uint64_t rev = reversed;
+    for(uint32_t k = 0; k < n; ++k)
     {
-        const uint64_t digit = inverse % base;
-        inverse = inverse / base;
-        index = index * base + digit;
+        // quotient and digit: the remainder before its correction is below
+        // 2 base, so it is exact modulo 2^24
+        uint32_t q = mulhi32(a, d.recip);
+        uint32_t i = (a - mul24(q, base)) & 0xffffffu;
+        if(i >= base)
+        {
+            i = i - base;
+            q = q + 1;
+        }
+        a = q;
+        const uint32_t p = (uint32_t)mix_bits(hash ^ rev);
+        const uint32_t p8 = p >> 8, p16 = p >> 16, p23 = p >> 23;
+        const uint32_t m27 = mul24(1u | p >> 27, 0x35fa69u);
+        do
+        {
+            i = i ^ p;
+            i = mul24(i, 0x70893du);
+            i = i ^ p16;
+            i = i ^ bit_field(i, 4, b4) ^ p8;
+            i = mul24(i, 0x29eb3fu);
+            i = i ^ p23;
+            i = i ^ bit_field(i, 1, b1);
+            i = mul24(i, m27);
+            i = i ^ bit_field(i, 11, b11);
+            i = mul24(i, 0xdcb303u);
+            i = i ^ bit_field(i, 2, b2);
+            i = mul24(i, 0x501cc3u);
+            i = i ^ bit_field(i, 2, b2);
+            i = mul24(i, 0x60a3dfu);
+            i = bit_field(i, 0, bits);
+            i = i ^ (i >> 5);
+        } while(i >= base);
+        // (i + p) mod base, again exact modulo 2^24 before the correction
+        const uint32_t x = i + p;
+        i = (x - mul24(mulhi32(x, d.recip), base)) & 0xffffffu;
+        if(i >= base)
+            i = i - base;
+        rev = (uint64_t)(uint32_t)rev * base + i;
     }
-    return index;
+    return rev;
+}
+
+// sample_halton (halton.cpp:39-44) of an index below 2^32 in two steps, so
+// that the table's load can be in flight while another dimension's digits
+// are computed: bit for bit owen_scrambled_radical_inverse
+struct HaltonDraw
+{
+    HaltonDim dim;
+    uint32_t high;     // index / span
+    uint32_t reversed; // the table's digits
+};
+
+BTRC_HD HaltonDraw halton_begin(const HaltonTables &tab, uint32_t dim, uint32_t index)
+{
+    HaltonDraw w;
+    w.dim = tab.dims[dim];
+    uint32_t low;
+    divmod_recip(index, w.dim.span, w.dim.span_recip, &w.high, &low);
+    w.reversed = tab.values[w.dim.first + low];
+    return w;
+}
+
+BTRC_HD float halton_end(const HaltonDraw &w)
+{
+    const uint64_t rev = halton_digits(w.dim, (w.dim.base >> 16) & 0xfu, w.high, w.reversed);
+    return fmin_(w.dim.scale * (float)rev, 0x1.fffffep-1f);
+}
+
+BTRC_HD float halton_value(const HaltonTables &tab, uint32_t dim, uint32_t index)
+{
+    return halton_end(halton_begin(tab, dim, index));
+}
+
+// the same without the table
+BTRC_HD float halton_value_digits(const HaltonTables &tab, uint32_t dim, uint32_t index)
+{
+    const HaltonDim d = tab.dims[dim];
+    const uint64_t rev = halton_digits(d, ((d.base >> 16) & 0xfu) + ((d.base >> 20) & 0x1fu), index, 0);
+    return fmin_(d.scale * (float)rev, 0x1.fffffep-1f);
+}
+
+// one entry of dimension d's table: the reversed digits of r < span
+BTRC_HD uint16_t halton_table_entry(const HaltonDim &d, uint32_t r)
+{
+    return (uint16_t)halton_digits(d, (d.base >> 20) & 0x1fu, r, 0);
 }
 
 // Per-film constants of the Halton sampler (initialize_consts, halton.cpp:118-133)
@@ -249,6 +340,8 @@ struct HaltonConsts
     int32_t base_scales[2];
     int32_t base_exponents[2];
     int32_t mult_inverse[2];
+    uint32_t offset_scale[2]; // (stride / base_scales[i]) * mult_inverse[i] mod stride
+    uint32_t stride;          // base_scales[0] * base_scales[1], at most 128 * 243
 };
 
 struct HaltonState
@@ -257,97 +350,46 @@ struct HaltonState
     uint64_t index;
 };
 
-// halton.cpp:39-44 (sample_halton); with tables (non-null values) the
-// first digits of the first HALTON_TABLE_DIMS dimensions come from them
-BTRC_HD float sample_halton(const int *primes, uint32_t dim, uint64_t halton_index,
-                            HaltonTables tab = HaltonTables{ nullptr, nullptr })
+// halton.cpp:39-44 (sample_halton)
+BTRC_HD float sample_halton(const int *primes, uint32_t dim, uint64_t halton_index)
 {
-    const uint64_t hash = mix_bits((uint64_t)(1u + (dim << 4)));
-    if(tab.values && dim < (uint32_t)HALTON_TABLE_DIMS)
-        return owen_scrambled_radical_inverse_tabled((uint32_t)primes[dim], halton_index, hash, tab.values,
-                                                     tab.dims[dim]);
-    return owen_scrambled_radical_inverse((uint32_t)primes[dim], halton_index, hash);
+    return owen_scrambled_radical_inverse((uint32_t)primes[dim], halton_index,
+                                          mix_bits((uint64_t)(1u + (dim << 4))));
 }
 
-// HaltonSampler(res, pixel, sample_index), halton.cpp:48-66
+// HaltonSampler(res, pixel, sample_index), halton.cpp:48-66. The pixel's
+// offset fits 32 bits: each inverse is below its scale (at most 243), each
+// offset_scale below the stride (at most 31,104).
 BTRC_HD HaltonState halton_start(const HaltonConsts &hc, uint32_t px, uint32_t py, int32_t sample_index)
 {
     HaltonState st;
     st.index = 0;
-    const int32_t sample_stride = hc.base_scales[0] * hc.base_scales[1];
-    if(sample_stride > 1)
+    if(hc.stride > 1)
     {
-        const uint32_t pm[2] = { px % MAX_HALTON_RESOLUTION, py % MAX_HALTON_RESOLUTION };
-        for(int i = 0; i < 2; ++i)
+        // inverse_radical_inverse (low_discrepancy.cpp:103-114) in bases 2 and 3
+        uint32_t x = px % MAX_HALTON_RESOLUTION, y = py % MAX_HALTON_RESOLUTION, ix = 0, iy = 0;
+        for(int i = 0; i < hc.base_exponents[0]; ++i)
         {
-            const uint64_t dim_offset = inverse_radical_inverse(
-                (uint64_t)pm[i], i == 0 ? 2u : 3u, hc.base_exponents[i]);
-            st.index = st.index + dim_offset * (uint64_t)(sample_stride / hc.base_scales[i])
-                                             * (uint64_t)hc.mult_inverse[i];
+            ix = ix * 2 + (x & 1u);
+            x = x >> 1;
         }
-        st.index = st.index % (uint64_t)sample_stride;
+        for(int i = 0; i < hc.base_exponents[1]; ++i)
+        {
+            iy = iy * 3 + y % 3;
+            y = y / 3;
+        }
+        st.index = (ix * hc.offset_scale[0] + iy * hc.offset_scale[1]) % hc.stride;
     }
-    st.index = st.index + (uint64_t)(sample_index * sample_stride);
+    st.index = st.index + (uint64_t)(int64_t)(int32_t)((uint32_t)sample_index * hc.stride);
     st.dimension = 2; // halton.cpp:64-65
     return st;
 }
 
-// get1d / get2d / get3d, halton.cpp:80-116
-BTRC_HD float halton_get1d(const int *primes, HaltonState &st, HaltonTables tab = HaltonTables{ nullptr, nullptr })
+// The dimension where a draw of n numbers (get1d, get2d, get3d,
+// halton.cpp:80-116) starts: back to 2 when it would pass the prime table
+BTRC_HD uint32_t halton_wrap(uint32_t dim, uint32_t n)
 {
-    if(st.dimension >= (uint32_t)PRIME_TABLE_SIZE)
-        st.dimension = 2;
-    const float r = sample_halton(primes, st.dimension, st.index, tab);
-    st.dimension = st.dimension + 1;
-    return r;
-}
-
-BTRC_HD void halton_get2d(const int *primes, HaltonState &st, float *a, float *b,
-                          HaltonTables tab = HaltonTables{ nullptr, nullptr })
-{
-    if(st.dimension + 1 >= (uint32_t)PRIME_TABLE_SIZE)
-        st.dimension = 2;
-    *a = sample_halton(primes, st.dimension, st.index, tab);
-    *b = sample_halton(primes, st.dimension + 1, st.index, tab);
-    st.dimension = st.dimension + 2;
-}
-
-BTRC_HD void halton_get3d(const int *primes, HaltonState &st, float *a, float *b, float *c,
-                          HaltonTables tab = HaltonTables{ nullptr, nullptr })
-{
-    if(st.dimension + 2 >= (uint32_t)PRIME_TABLE_SIZE)
-        st.dimension = 2;
-    *a = sample_halton(primes, st.dimension, st.index, tab);
-    *b = sample_halton(primes, st.dimension + 1, st.index, tab);
-    *c = sample_halton(primes, st.dimension + 2, st.index, tab);
-    st.dimension = st.dimension + 3;
-}
-
-// one dimension's table (host side): the reversed digits after the first
-// info.digits steps for every a < info.span
-BTRC_HD void fill_halton_table(uint32_t base, uint32_t dim, HaltonDim info, uint16_t *out)
-{
-    const uint64_t hash = mix_bits((uint64_t)(1u + (dim << 4)));
-    const uint32_t m = 0xffffffffu / base, w = permutation_mask(base);
-    for(uint32_t r = 0; r < info.span; ++r)
-    {
-        uint64_t a = r, reversed = 0;
-        for(uint32_t j = 0; j < info.digits; ++j)
-            reversed = owen_digit(base, m, w, hash, a, reversed);
-        out[r] = (uint16_t)reversed;
-    }
-}
-
-// K and base^K of a base's table: the most digits with base^K <= HALTON_TABLE_SPAN
-BTRC_HD HaltonDim halton_dim_shape(uint32_t base, uint32_t first)
-{
-    uint32_t span = 1, k = 0;
-    while(span * base <= HALTON_TABLE_SPAN)
-    {
-        span *= base;
-        ++k;
-    }
-    return HaltonDim{ first, span, k, 0xffffffffu / span };
+    return dim + n > (uint32_t)PRIME_TABLE_SIZE ? 2u : dim;
 }
 
 // ---- independent sampler

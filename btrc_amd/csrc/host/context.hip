@@ -193,6 +193,9 @@ HaltonConsts make_halton_consts(int32_t width, int32_t height)
     }
     hc.mult_inverse[0] = (int32_t)multiplicative_inverse(hc.base_scales[1], hc.base_scales[0]);
     hc.mult_inverse[1] = (int32_t)multiplicative_inverse(hc.base_scales[0], hc.base_scales[1]);
+    hc.stride = (uint32_t)(hc.base_scales[0] * hc.base_scales[1]);
+    for(int i = 0; i < 2; ++i)
+        hc.offset_scale[i] = (uint32_t)((hc.stride / (uint32_t)hc.base_scales[i]) * (uint32_t)hc.mult_inverse[i] % hc.stride);
     return hc;
 }
 
@@ -1701,25 +1704,25 @@ void nrc_collect(btrc_ctx *ctx, int32_t steps)
     n.last = r;
 }
 
-// the Halton sampler's first-digit tables in device memory (a pure function
-// of the prime table: 226,691 values, 443 KB)
+// the Halton sampler's dimensions and first-digit tables in device memory (a
+// pure function of the prime table: 5.0 million values, 10 MB, made by a
+// kernel on first use)
 HaltonTables halton_tables(btrc_ctx *ctx)
 {
     if(!ctx->halton_values.ptr)
     {
         constexpr PrimeTable primes = make_prime_table();
-        std::vector<HaltonDim> dims(HALTON_TABLE_DIMS);
+        std::vector<HaltonDim> dims(PRIME_TABLE_SIZE);
         uint32_t total = 0;
-        for(int d = 0; d < HALTON_TABLE_DIMS; ++d)
+        for(int d = 0; d < PRIME_TABLE_SIZE; ++d)
         {
-            dims[d] = halton_dim_shape((uint32_t)primes.p[d], total);
+            dims[d] = halton_dim((uint32_t)primes.p[d], (uint32_t)d, total);
             total += dims[d].span;
         }
-        std::vector<uint16_t> values(total);
-        for(int d = 0; d < HALTON_TABLE_DIMS; ++d)
-            fill_halton_table((uint32_t)primes.p[d], (uint32_t)d, dims[d], values.data() + dims[d].first);
         ctx->halton_dims.upload(dims.data(), dims.size(), ctx->stream);
-        ctx->halton_values.upload(values.data(), values.size(), ctx->stream);
+        ctx->halton_values.alloc(total);
+        launch_halton_tables(ctx->stream, ctx->halton_dims.ptr, PRIME_TABLE_SIZE, ctx->halton_values.ptr);
+        BTRC_HIP_CHECK(hipGetLastError());
         BTRC_HIP_CHECK(hipStreamSynchronize(ctx->stream));
     }
     return HaltonTables{ ctx->halton_values.ptr, ctx->halton_dims.ptr };

@@ -22,7 +22,7 @@ struct PathSOA
     float4 *beta;     // throughput.xyz, depth bits
     float4 *rad;      // path radiance.xyz, training path id bits (cache mode) or ~0
     float4 *bsdf_le;  // beta_le.xyz, bsdf pdf (negative: delta lobe)
-    uint4 *smp;       // pixel index, then Halton: dimension, index lo, hi;
+    uint4 *smp;       // pixel index, then Halton: dimension, index, 0;
                       // independent: PCG state lo, hi, unused
 };
 
@@ -209,7 +209,7 @@ struct RenderConsts
     // paths with id pixel / nrc_stride while that is below nrc_max_paths
     int32_t nrc_stride, nrc_phase, nrc_max_paths;
     FilterConsts filter;
-    HaltonTables halton;    // first-digit tables of the Halton sampler
+    HaltonTables halton;    // dimensions and first-digit tables of the Halton sampler
 };
 
 // the view holding film pixel `pixel`
@@ -289,6 +289,8 @@ void launch_envir_table(hipStream_t s, const TextureView &tv, int32_t tex, int32
 // the environment light's eval_le, pdf_li and sample_li: 12 floats per query
 void launch_envir_eval(hipStream_t s, const SceneView &sv, const float *dirs, const float *sam, int32_t n, float *out);
 void launch_texture_eval(hipStream_t s, const TextureView &tv, int32_t id, const float2 *uv, int32_t n, float4 *out);
+// the Halton sampler's first-digit tables of `count` dimensions
+void launch_halton_tables(hipStream_t s, const HaltonDim *dims, int32_t count, uint16_t *values);
 void launch_volume_eval(hipStream_t s, const VolumeView &vv, const float4 *seg, const uint2 *seed, int32_t n,
                         float *out);
 void launch_medium_eval(hipStream_t s, const SceneView &sv, int32_t med, const float4 *seg, const uint2 *seed,

@@ -81,30 +81,77 @@ __device__ __forceinline__ void aov_splat(float *buf, uint32_t pixel, V3 v)
 __device__ __forceinline__ V3 xyz(float4 a) { return v3(a.x, a.y, a.z); }
 __device__ __forceinline__ float4 f4(V3 a, float w) { return make_float4(a.x, a.y, a.z, w); }
 
+// A pointer loaded from a device-memory record, known to be global: without
+// this its loads compile to flat ones, which also wait on the LDS counter
+template<class T> __device__ __forceinline__ const T *as_global(const T *p)
+{
+    return (const T *)(const __attribute__((address_space(1))) T *)p;
+}
+
+__device__ __forceinline__ HaltonTables global_tables(const HaltonTables &t)
+{
+    return HaltonTables{ as_global(t.values), as_global(t.dims) };
+}
+
+// A surface or scattering vertex draws its light sample (three numbers), its
+// light (one) and its continuation (three), in this order
+constexpr int VERTEX_DRAWS = 7;
+
 // The sampler of a path, kept in PathSOA::smp between stages (x = pixel).
 template<int SAMPLER> struct PathSampler;
 
 template<> struct PathSampler<SAMPLER_HALTON>
 {
-    HaltonState st;
+    HaltonTables tab;
+    uint32_t dimension;
+    uint32_t index; // below 2^31 (render's limit on samples times stride)
 
-    __device__ static PathSampler start(const ViewRec &view, uint32_t px, uint32_t py, int32_t sample)
+    __device__ static PathSampler start(const RenderConsts &rc, const ViewRec &view, uint32_t px, uint32_t py,
+                                        int32_t sample)
     {
-        return PathSampler{ halton_start(view.halton, px, py, sample) };
+        const HaltonState st = halton_start(view.halton, px, py, sample);
+        return PathSampler{ global_tables(rc.halton), st.dimension, (uint32_t)st.index };
     }
-    __device__ static PathSampler load(const RenderConsts &, uint4 s)
+    __device__ static PathSampler load(const RenderConsts &rc, uint4 s) { return PathSampler{ global_tables(rc.halton), s.y, s.z }; }
+    __device__ uint4 pack(uint32_t pixel) const { return make_uint4(pixel, dimension, index, 0u); }
+    __device__ float get1d()
     {
-        PathSampler r;
-        r.st.dimension = s.y;
-        r.st.index = (uint64_t)s.z | ((uint64_t)s.w << 32);
-        return r;
+        const uint32_t dim = halton_wrap(dimension, 1);
+        dimension = dim + 1;
+        return halton_value(tab, dim, index);
     }
-    __device__ uint4 pack(uint32_t pixel) const
+    // the same by the digit loop alone: in k_medium_track every lane is at a
+    // dimension of its own, hundreds into the sequence, so the lookups miss
+    // the L2 and each tracking step would wait for two of them (media frame,
+    // 1080p at 4 spp: 52.1 ms of tracking with the tables, 46.0 without)
+    __device__ float get1d_digits()
     {
-        return make_uint4(pixel, st.dimension, (uint32_t)st.index, (uint32_t)(st.index >> 32));
+        const uint32_t dim = halton_wrap(dimension, 1);
+        dimension = dim + 1;
+        return halton_value_digits(tab, dim, index);
     }
-    __device__ float get1d() { return halton_get1d(c_primes.p, st); }
-    __device__ void get3d(float *a, float *b, float *c) { halton_get3d(c_primes.p, st, a, b, c); }
+    // a vertex's draws into u[0], u[stride], ...: one copy of the digit loop,
+    // each dimension's table lookup in flight while the previous one's digits
+    // are computed
+    __device__ void vertex_draws(float *u, int stride)
+    {
+        uint32_t dim = halton_wrap(dimension, 3);
+        HaltonDraw next = halton_begin(tab, dim, index);
+#pragma unroll 1
+        for(int k = 0; k < VERTEX_DRAWS; ++k)
+        {
+            const HaltonDraw cur = next;
+            dim = dim + 1;
+            if(k == 2)
+                dim = halton_wrap(dim, 1);
+            if(k == 3)
+                dim = halton_wrap(dim, 3);
+            if(k + 1 < VERTEX_DRAWS)
+                next = halton_begin(tab, dim, index);
+            u[k * stride] = halton_end(cur);
+        }
+        dimension = dim;
+    }
 };
 
 // Sampler::get2d/get3d default to consecutive get1d (core/sampler.h:15-28);
@@ -113,7 +160,8 @@ template<> struct PathSampler<SAMPLER_INDEPENDENT>
 {
     Pcg32 rng;
 
-    __device__ static PathSampler start(const ViewRec &, uint32_t px, uint32_t py, int32_t sample)
+    __device__ static PathSampler start(const RenderConsts &, const ViewRec &, uint32_t px, uint32_t py,
+                                        int32_t sample)
     {
         return PathSampler{ independent_start(px, py, sample) };
     }
@@ -132,46 +180,10 @@ template<> struct PathSampler<SAMPLER_INDEPENDENT>
         return make_uint4(pixel, (uint32_t)rng.state, (uint32_t)(rng.state >> 32), 0u);
     }
     __device__ float get1d() { return pcg32_uniform_float(rng); }
-    __device__ void get3d(float *a, float *b, float *c)
+    __device__ void vertex_draws(float *u, int stride)
     {
-        *a = get1d();
-        *b = get1d();
-        *c = get1d();
-    }
-};
-
-// generate's sampler: the Halton sampler reads the camera samples' first
-// digits from the first-digit tables (same values). The later stages run
-// the digit loop alone: in shade and k_medium_scatter the lookups cost more
-// registers than they save, and in k_medium_track (two draws per tracking
-// step) the dependent table loads cost more time than the digits they save.
-template<int SAMPLER> struct TabledSampler
-{
-    PathSampler<SAMPLER> smp;
-
-    __device__ static TabledSampler start(const RenderConsts &, const ViewRec &view, uint32_t px, uint32_t py,
-                                          int32_t sample)
-    {
-        return TabledSampler{ PathSampler<SAMPLER>::start(view, px, py, sample) };
-    }
-    __device__ float get1d() { return smp.get1d(); }
-    __device__ uint4 pack(uint32_t pixel) const { return smp.pack(pixel); }
-};
-
-template<> struct TabledSampler<SAMPLER_HALTON>
-{
-    HaltonState st;
-    HaltonTables tab;
-
-    __device__ static TabledSampler start(const RenderConsts &rc, const ViewRec &view, uint32_t px, uint32_t py,
-                                          int32_t sample)
-    {
-        return TabledSampler{ halton_start(view.halton, px, py, sample), rc.halton };
-    }
-    __device__ float get1d() { return halton_get1d(c_primes.p, st, tab); }
-    __device__ uint4 pack(uint32_t pixel) const
-    {
-        return PathSampler<SAMPLER_HALTON>{ st }.pack(pixel);
+        for(int k = 0; k < VERTEX_DRAWS; ++k)
+            u[k * stride] = get1d();
     }
 };
 
@@ -255,18 +267,21 @@ __global__ void __launch_bounds__(256) k_generate(const RenderConsts *__restrict
         const uint64_t pixels = (uint64_t)view.width * (uint64_t)view.height;
         // generate.cpp:46-62: uniform order walks all pixels once per sample
         // index; tile order finishes a pixel's samples before the next pixel
-        uint32_t local_pixel;
-        int32_t sample_index;
-        if(rc.tile)
+        const uint64_t divisor = rc.tile ? (uint64_t)rc.spp : pixels;
+        uint64_t quo, rem;
+        if((local | divisor) >> 32 == 0)
         {
-            local_pixel = (uint32_t)(local / (uint64_t)rc.spp);
-            sample_index = (int32_t)(local % (uint64_t)rc.spp);
+            // a 64-bit division costs as much as a Halton dimension
+            quo = (uint32_t)local / (uint32_t)divisor;
+            rem = (uint32_t)local - (uint32_t)quo * (uint32_t)divisor;
         }
         else
         {
-            local_pixel = (uint32_t)(local % pixels);
-            sample_index = (int32_t)(local / pixels);
+            quo = local / divisor;
+            rem = local - quo * divisor;
         }
+        const uint32_t local_pixel = (uint32_t)(rc.tile ? quo : rem);
+        int32_t sample_index = (int32_t)(rc.tile ? rem : quo);
         sample_index += rc.sample_offset;
         const uint32_t pixel_index = view.pixel_base + local_pixel; // film pixel
         uint32_t train = NO_TRAIN;
@@ -276,7 +291,7 @@ __global__ void __launch_bounds__(256) k_generate(const RenderConsts *__restrict
         const uint32_t px = local_pixel % (uint32_t)view.width;
         const uint32_t py = local_pixel / (uint32_t)view.width;
 
-        TabledSampler<SAMPLER> smp = TabledSampler<SAMPLER>::start(rc, view, px, py, sample_index);
+        PathSampler<SAMPLER> smp = PathSampler<SAMPLER>::start(rc, view, px, py, sample_index);
         float fx, fy;
         if(rc.filter.type == FILTER_GAUSSIAN)
         {
@@ -397,6 +412,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))
     const RenderConsts *__restrict__ rcp, SceneView sv, WaveCounters *c, PathSOA path, HitSOA hit,
     PathSOA next, ShadowSOA shadow, FilmView film, NrcView nrc, int parity)
 {
+    __shared__ float s_draws[VERTEX_DRAWS * 256];
+    float *u = s_draws + threadIdx.x; // the lane's draws, 256 apart
     const RenderConsts &rc = *rcp;
     QueueState *q = queue_state(c);
     const int32_t n = c->active;
@@ -414,20 +431,54 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))
         {
             const int32_t ps = pool_slot(q, w0, i); // the state's pool slot
             const uint32_t flag = hit.flag[i];
-            const float4 ro = path.ray_o[ps];
-            const float4 rd = path.ray_d[ps];
             const float4 beta_depth = path.beta[ps];
             const float4 rad4 = path.rad[ps];
-            const float4 le4 = path.bsdf_le[ps];
             const uint4 smp = path.smp[ps];
             const uint32_t pixel = smp.x;
             PathSampler<SAMPLER> hs = PathSampler<SAMPLER>::load(rc, smp);
 
-            const V3 o = xyz(ro), d = xyz(rd);
             V3 beta = xyz(beta_depth);
             const int32_t depth = __float_as_int(beta_depth.w);
             V3 path_rad = xyz(rad4);
             const uint32_t train = __float_as_uint(rad4.w);
+            // whether the cache answers for the rest of this path at this
+            // vertex (a training path's tail, or a rendered path's prefix)
+            const bool cache_end = train != NO_TRAIN ? depth == nrc.train_depth && nrc.queries != nullptr
+                                                     : depth == nrc.query_depth;
+
+            // Every number the vertex draws, before anything else is live:
+            // the digit loops run with the fewest registers and no spills.
+            // Russian roulette (simple_russian_roulette, helper.cpp:67-97)
+            // looks at the throughput only, so it is decided here too.
+            bool rr_exit = false;
+            V3 beta_rr = beta;
+            if((flag & (PATH_FLAG_HAS_INTERSECTION | PATH_FLAG_HAS_SCATTERING)) == PATH_FLAG_HAS_INTERSECTION &&
+               !cache_end)
+            {
+                if(depth >= rc.min_depth)
+                {
+                    if(depth >= rc.max_depth)
+                        rr_exit = true;
+                    else
+                    {
+                        const float rr = hs.get1d();
+                        if(luminance(beta) < rc.rr_threshold)
+                        {
+                            if(rr > rc.rr_cont_prob)
+                                rr_exit = true;
+                            else
+                                beta_rr = beta / rc.rr_cont_prob;
+                        }
+                    }
+                }
+                if(!rr_exit)
+                    hs.vertex_draws(u, 256);
+            }
+
+            const float4 ro = path.ray_o[ps];
+            const float4 rd = path.ray_d[ps];
+            const float4 le4 = path.bsdf_le[ps];
+            const V3 o = xyz(ro), d = xyz(rd);
             const V3 beta_le = xyz(le4);
             const float bsdf_pdf = le4.w;
 
@@ -461,7 +512,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))
                     // record (throughput before Russian roulette, so that the
                     // target stays unbiased)
                     train_add(nrc.acc, train, le_rad);
-                    if(depth == nrc.train_depth && nrc.queries)
+                    if(cache_end)
                     {
                         // self-training: the cache answers for the tail of
                         // the training path; its answer joins the path's sum
@@ -485,7 +536,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))
                         r.valid = 1;
                     }
                 }
-                else if(!done && depth == nrc.query_depth)
+                else if(!done && cache_end)
                 {
                     // the prefix ends here: the cache answers for the rest
                     if(nrc.queries)
@@ -503,24 +554,6 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))
                 if(!done)
                 {
                     path_rad = path_rad + le_rad;
-                    // simple_russian_roulette, helper.cpp:67-97
-                    bool rr_exit = false;
-                    if(depth >= rc.min_depth)
-                    {
-                        if(depth >= rc.max_depth)
-                            rr_exit = true;
-                        else
-                        {
-                            const float u = hs.get1d();
-                            if(luminance(beta) < rc.rr_threshold)
-                            {
-                                if(u > rc.rr_cont_prob)
-                                    rr_exit = true;
-                                else
-                                    beta = beta / rc.rr_cont_prob;
-                            }
-                        }
-                    }
                     if(rr_exit)
                     {
                         film_splat(film, pixel, path_rad);
@@ -529,10 +562,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))
                 }
                 if(!done)
                 {
-                    float l0, l1, l2;
-                    hs.get3d(&l0, &l1, &l2);
-                    const float lsel = hs.get1d();
-                    ShadowSample ss = sample_surface_light_li(sv, sp.position, sp.frame.z, l0, l1, l2, lsel);
+                    beta = beta_rr;
+                    ShadowSample ss = sample_surface_light_li(sv, sp.position, sp.frame.z, u[0], u[256], u[2 * 256],
+                                                              u[3 * 256]);
 
                     const Shader shader = make_shader(material_at(sv, inst.material_id, sp), sp.frame, sp.interp_z);
                     if(depth == 0)
@@ -544,11 +576,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))
                         if(film.normal)
                             aov_splat(film.normal, pixel, shader_normal(shader));
                     }
-                    // draws in the reference's order; the light connection
-                    // is finished (its shadow ray pushed) before the BSDF is
-                    // sampled, then the continuation
-                    float s0, s1, s2;
-                    hs.get3d(&s0, &s1, &s2);
+                    // the light connection is finished (its shadow ray
+                    // pushed) before the BSDF is sampled, then the
+                    // continuation
                     V3 shadow_f = v3s(0.0f);
                     float shadow_pdf = 0.0f;
                     if(ss.success)
@@ -578,7 +608,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))
                     }
 
                     BSDFSample bs;
-                    shader_sample(shader, -d, s0, s1, s2, bs);
+                    shader_sample(shader, -d, u[4 * 256], u[5 * 256], u[6 * 256], bs);
                     if(!is_zero(bs.bsdf))
                     {
                         const V3 dir = normalize(bs.dir);
@@ -660,6 +690,19 @@ __device__ __forceinline__ void record_scatter(float4 *scatter, int32_t i, const
     scatter[2 * (size_t)i + 1] = f4(ms.color, 0.0f);
 }
 
+// the tracking loop's draws (PathSampler::get1d_digits)
+template<int SAMPLER> struct TrackSampler
+{
+    PathSampler<SAMPLER> path;
+    __device__ float get1d() { return path.get1d(); }
+};
+
+template<> struct TrackSampler<SAMPLER_HALTON>
+{
+    PathSampler<SAMPLER_HALTON> path;
+    __device__ float get1d() { return path.get1d_digits(); }
+};
+
 template<int SAMPLER>
 __global__ void __launch_bounds__(MEDIUM_BLOCK) k_medium_track(const RenderConsts *__restrict__ rcp, SceneView sv,
                                                                WaveCounters *c, PathSOA path, HitSOA hit,
@@ -690,7 +733,7 @@ __global__ void __launch_bounds__(MEDIUM_BLOCK) k_medium_track(const RenderConst
     bool active = false, sampling = false, scattered = false;
     int32_t i = 0, ps = 0;
     uint32_t flag = 0, pixel = 0, med = 0;
-    PathSampler<SAMPLER> hs{};
+    TrackSampler<SAMPLER> hs{};
     GridTrack g{};
     float tr = 1.0f;
 
@@ -778,7 +821,7 @@ __global__ void __launch_bounds__(MEDIUM_BLOCK) k_medium_track(const RenderConst
                     const V3 end = v3(q_end[0][e], q_end[1][e], q_end[2][e]);
                     const uint4 smp = path.smp[ps];
                     pixel = smp.x;
-                    hs = PathSampler<SAMPLER>::load(rc, smp);
+                    hs.path = PathSampler<SAMPLER>::load(rc, smp);
                     g = grid_track_start(sv.media[med], o, end);
                     tr = 1.0f;
                     sampling = true;
@@ -831,7 +874,7 @@ __global__ void __launch_bounds__(MEDIUM_BLOCK) k_medium_track(const RenderConst
             {
                 const float4 le4 = path.bsdf_le[ps];
                 path.bsdf_le[ps] = f4(xyz(le4) * v3s(tr), le4.w);
-                path.smp[ps] = hs.pack(pixel);
+                path.smp[ps] = hs.path.pack(pixel);
                 if(scattered)
                     hit.flag[i] = flag | PATH_FLAG_HAS_SCATTERING;
                 active = false;
@@ -848,6 +891,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))
     const RenderConsts *__restrict__ rcp, SceneView sv, WaveCounters *c, PathSOA path, HitSOA hit,
     const float4 *scatter, PathSOA next, ShadowSOA shadow, FilmView film, int parity)
 {
+    __shared__ float s_draws[VERTEX_DRAWS * 256];
+    float *u = s_draws + threadIdx.x; // the lane's draws, 256 apart
     const RenderConsts &rc = *rcp;
     QueueState *q = queue_state(c);
     const int32_t n = c->active;
@@ -927,10 +972,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))
                     rr_exit = true;
                 else
                 {
-                    const float u = hs.get1d();
+                    const float rr = hs.get1d();
                     if(luminance(beta) < rc.rr_threshold)
                     {
-                        if(u > rc.rr_cont_prob)
+                        if(rr > rc.rr_cont_prob)
                             rr_exit = true;
                         else
                             beta = beta / rc.rr_cont_prob;
@@ -941,19 +986,16 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))
                 film_splat(film, pixel, path_rad);
             else
             {
-                float l0, l1, l2;
-                hs.get3d(&l0, &l1, &l2);
-                const float lsel = hs.get1d();
-                ShadowSample ss = sample_light_li(sv, position, v3s(0.0f), false, l0, l1, l2, lsel);
+                hs.vertex_draws(u, 256);
+                ShadowSample ss = sample_light_li(sv, position, v3s(0.0f), false, u[0], u[256], u[2 * 256],
+                                                  u[3 * 256]);
                 V3 beta_li = v3s(0.0f);
                 if(ss.success)
                 {
                     const float pv = hg_pdf(gph, ss.d, -d);
                     beta_li = ss.li * beta * (color * pv) / (pv + ss.light_pdf);
                 }
-                float s0, s1, s2;
-                hs.get3d(&s0, &s1, &s2);
-                const PhaseSample phs = hg_sample(gph, color, -d, s0, s1);
+                const PhaseSample phs = hg_sample(gph, color, -d, u[4 * 256], u[5 * 256]);
                 if(ss.success)
                 {
                     const uint32_t smed = ss.t1 > 1.0f ? (uint32_t)sv.medium_count : med;
@@ -1282,12 +1324,25 @@ __global__ void k_halton_eval(HaltonConsts hc, HaltonTables tab, const uint32_t 
     const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if(i >= n)
         return;
-    // even samples read the first-digit tables, odd ones run the digit loop
-    // alone (the camera samples and the later stages' forms)
-    const HaltonTables t = (i & 1) ? HaltonTables{ nullptr, nullptr } : tab;
+    // even samples as the stages evaluate them (tables, 32-bit indices), odd
+    // ones and indices beyond 32 bits by the digit loop alone
     HaltonState hs = halton_start(hc, px[i], py[i], si[i]);
+    const bool tabled = !(i & 1) && (hs.index >> 32) == 0;
     for(int32_t k = 0; k < dims; ++k)
-        out[(size_t)i * dims + k] = halton_get1d(c_primes.p, hs, t);
+    {
+        const uint32_t dim = halton_wrap(hs.dimension, 1);
+        out[(size_t)i * dims + k] = tabled ? halton_value(tab, dim, (uint32_t)hs.index)
+                                           : sample_halton(c_primes.p, dim, hs.index);
+        hs.dimension = dim + 1;
+    }
+}
+
+// the first-digit tables, one workgroup row per dimension
+__global__ void k_halton_tables(const HaltonDim *dims, uint16_t *values)
+{
+    const HaltonDim d = dims[blockIdx.y];
+    for(uint32_t r = blockIdx.x * blockDim.x + threadIdx.x; r < d.span; r += gridDim.x * blockDim.x)
+        values[d.first + r] = halton_table_entry(d, r);
 }
 
 // ACESToneMap's kernel, postprocess/tonemap.cpp:14-24,35-51: Narkowicz's
@@ -1482,6 +1537,11 @@ void launch_halton_eval(hipStream_t s, const HaltonConsts &hc, const HaltonTable
 {
     hipLaunchKernelGGL(k_halton_eval, dim3((n + 127) / 128), dim3(128), 0, s, hc, tab, px, py, sample_index, n, dims,
                        out);
+}
+
+void launch_halton_tables(hipStream_t s, const HaltonDim *dims, int32_t count, uint16_t *values)
+{
+    hipLaunchKernelGGL(k_halton_tables, dim3(16, count), dim3(256), 0, s, dims, values);
 }
 
 void launch_volume_eval(hipStream_t s, const VolumeView &vv, const float4 *seg, const uint2 *seed, int32_t n,
