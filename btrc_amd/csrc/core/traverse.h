@@ -40,73 +40,69 @@ struct alignas(16) BvhNode4
 };
 static_assert(sizeof(BvhNode4) == 128, "BvhNode4 must be one 128-byte line");
 
+// A ray as the slab test reads it: the distance to a plane is one fused
+// multiply-add b * inv + c, with the rounding of c paid for in advance.
 struct RayBoxPre
 {
-    V3 o;
-    V3 inv;      // 1 / d
-    V3 inv_pad;  // 1 / d enlarged by 2 ulps (Ize, "Robust BVH Ray Traversal", JCGT 2013)
+    V3 inv;   // 1 / d, at most 2^96 in magnitude
+    V3 near_c; // -o / d, lowered: entry distances never come out late
+    V3 far_c;  // -o / d, raised: exit distances never come out early
     bool neg_x, neg_y, neg_z;
 };
 
-BTRC_HD float add_ulp_magnitude(float x, uint32_t ulps)
+// One axis. With inv = 1/d (1 + e1) and oi = o inv (1 + e2), |e| <= 2^-24,
+// the plane distance fma(b, inv, -oi) differs from (b - o) / d by at most
+// 2^-23 of itself plus 2^-24 |oi|. near_c and far_c move by 2^-22 |oi| (and
+// their own rounding takes at most 2^-24 of it), so only the relative part is
+// left, which raybox_nf pays on the exit side. Directions of magnitude below
+// 2^-96 (zero among them) count as 2^-96: their planes lie beyond every
+// scene, and the 2^-80 |inv| term keeps a ray that runs inside a plane of the
+// box (o on it, d zero) inside the box.
+BTRC_HD void raybox_axis(float o, float d, float *inv, float *near_c, float *far_c)
 {
-    return isfinite_(x) ? u2f(f2u(x) + ulps) : x;
+    const float big = 7.9228163e28f; // 2^96
+    const float m = fmaxf(fminf(fabsf(1.0f / d), big), 1.1754944e-38f); // never 0: an empty slot's planes stay infinite
+    const float v = u2f(f2u(m) | (f2u(d) & 0x80000000u));
+    const float oi = o * v;
+    const float up = 1.0f + 2.3841858e-7f, down = 1.0f - 2.3841858e-7f; // 1 +- 2^-22
+    const float tiny = m * 8.2718061e-25f;                              // 2^-80 |inv|
+    *inv = v;
+    *near_c = -(oi * (oi > 0.0f ? up : down)) - tiny;
+    *far_c = -(oi * (oi > 0.0f ? down : up)) + tiny;
 }
 
 BTRC_HD RayBoxPre raybox_pre(V3 o, V3 d)
 {
     RayBoxPre p;
-    p.o = o;
-    p.inv = v3(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
-    p.inv_pad = v3(add_ulp_magnitude(p.inv.x, 2), add_ulp_magnitude(p.inv.y, 2), add_ulp_magnitude(p.inv.z, 2));
+    raybox_axis(o.x, d.x, &p.inv.x, &p.near_c.x, &p.far_c.x);
+    raybox_axis(o.y, d.y, &p.inv.y, &p.near_c.y, &p.far_c.y);
+    raybox_axis(o.z, d.z, &p.inv.z, &p.near_c.z, &p.far_c.z);
     p.neg_x = (f2u(d.x) >> 31) != 0;
     p.neg_y = (f2u(d.y) >> 31) != 0;
     p.neg_z = (f2u(d.z) >> 31) != 0;
     return p;
 }
 
-// robust_max / robust_min (lib/bvh/include/bvh/utilities.hpp:62-71): a NaN on
-// the left is dropped in favour of the right operand
-BTRC_HD float rmax(float a, float b) { return a > b ? a : b; }
-BTRC_HD float rmin(float a, float b) { return a < b ? a : b; }
-
-// The slab test with the near and far planes already chosen by the ray's
-// direction signs; same arithmetic as raybox.
+// Conservative slab test of one box, its near and far planes already chosen
+// by the ray's direction signs; the entry distance goes to *tentry. Six
+// fused multiply-adds: half the arithmetic of (b - o) * inv per plane. The
+// maxNum / minNum chains drop NaN operands (0 * inf planes), as the robust
+// max / min of lib/bvh do (lib/bvh/include/bvh/utilities.hpp:62-71); tmin and
+// tmax are never NaN. The exit side is widened by 2^-21, more than the two
+// sides' 2^-23 each (Ize, "Robust BVH Ray Traversal", JCGT 2013).
 BTRC_HD bool raybox_nf(const RayBoxPre &p, float nx, float fx, float ny, float fy, float nz, float fz,
                        float tmin, float tmax, float *tentry)
 {
-    const float t0x = (nx - p.o.x) * p.inv.x;
-    const float t0y = (ny - p.o.y) * p.inv.y;
-    const float t0z = (nz - p.o.z) * p.inv.z;
-    const float t1x = (fx - p.o.x) * p.inv_pad.x;
-    const float t1y = (fy - p.o.y) * p.inv_pad.y;
-    const float t1z = (fz - p.o.z) * p.inv_pad.z;
+    const float t0x = fmaf(nx, p.inv.x, p.near_c.x);
+    const float t0y = fmaf(ny, p.inv.y, p.near_c.y);
+    const float t0z = fmaf(nz, p.inv.z, p.near_c.z);
+    const float t1x = fmaf(fx, p.inv.x, p.far_c.x);
+    const float t1y = fmaf(fy, p.inv.y, p.far_c.y);
+    const float t1z = fmaf(fz, p.inv.z, p.far_c.z);
     const float te = fmaxf(t0x, fmaxf(t0y, fmaxf(t0z, tmin)));
     const float tx = fminf(t1x, fminf(t1y, fminf(t1z, tmax)));
     *tentry = te;
-    return te <= tx;
-}
-
-// Conservative slab test of one box; returns the entry distance through *tentry.
-BTRC_HD bool raybox(const RayBoxPre &p, float lox, float hix, float loy, float hiy, float loz, float hiz,
-                    float tmin, float tmax, float *tentry)
-{
-    const float nx = p.neg_x ? hix : lox, fx = p.neg_x ? lox : hix;
-    const float ny = p.neg_y ? hiy : loy, fy = p.neg_y ? loy : hiy;
-    const float nz = p.neg_z ? hiz : loz, fz = p.neg_z ? loz : hiz;
-    const float t0x = (nx - p.o.x) * p.inv.x;
-    const float t0y = (ny - p.o.y) * p.inv.y;
-    const float t0z = (nz - p.o.z) * p.inv.z;
-    const float t1x = (fx - p.o.x) * p.inv_pad.x;
-    const float t1y = (fy - p.o.y) * p.inv_pad.y;
-    const float t1z = (fz - p.o.z) * p.inv_pad.z;
-    // robust max / min: tmin and tmax are never NaN, so every right operand
-    // of the chains is a number and IEEE maxNum / minNum (which drop a NaN
-    // operand) give exactly rmax / rmin, in fewer instructions
-    const float te = fmaxf(t0x, fmaxf(t0y, fmaxf(t0z, tmin)));
-    const float tx = fminf(t1x, fminf(t1y, fminf(t1z, tmax)));
-    *tentry = te;
-    return te <= tx;
+    return te <= fmaf(fabsf(tx), 4.7683716e-7f, tx);
 }
 
 // Box culling distance for the current closest hit. A box's entry distance
@@ -132,17 +128,19 @@ BTRC_HD float cull_distance(float best_t, float margin)
 
 // ---- watertight test ----
 
+// The ray as the watertight test reads it: its axes permuted so that z is the
+// largest direction component, and the shear to it. Triangle coordinates
+// come in the same permutation.
 struct WatertightPre
 {
-    V3 o;
     int32_t kx, ky, kz;
+    float ox, oy, oz; // origin components kx, ky, kz
     float Sx, Sy, Sz;
 };
 
 BTRC_HD WatertightPre watertight_pre(V3 o, V3 d)
 {
     WatertightPre w;
-    w.o = o;
     const float ax = fabs_(d.x), ay = fabs_(d.y), az = fabs_(d.z);
     int32_t kz = ax > ay ? (ax > az ? 0 : 2) : (ay > az ? 1 : 2);
     int32_t kx = kz + 1 == 3 ? 0 : kz + 1;
@@ -156,6 +154,9 @@ BTRC_HD WatertightPre watertight_pre(V3 o, V3 d)
     w.kx = kx;
     w.ky = ky;
     w.kz = kz;
+    w.ox = comp(o, kx);
+    w.oy = comp(o, ky);
+    w.oz = comp(o, kz);
     const float dz = comp(d, kz);
     w.Sx = comp(d, kx) / dz;
     w.Sy = comp(d, ky) / dz;
@@ -164,20 +165,17 @@ BTRC_HD WatertightPre watertight_pre(V3 o, V3 d)
 }
 
 // Returns true on a hit with t in [tmin, tmax]; (b1, b2) are the barycentric
-// weights of v1 and v2.
-BTRC_HD bool watertight_hit(const WatertightPre &w, V3 v0, V3 v1, V3 v2, float tmin, float tmax,
+// weights of v1 and v2. vx, vy, vz: components kx, ky, kz of v0, v1, v2.
+BTRC_HD bool watertight_hit(const WatertightPre &w, V3 vx, V3 vy, V3 vz, float tmin, float tmax,
                             float *t_out, float *b1_out, float *b2_out)
 {
-    const V3 A = v0 - w.o;
-    const V3 B = v1 - w.o;
-    const V3 C = v2 - w.o;
-    const float Akz = comp(A, w.kz), Bkz = comp(B, w.kz), Ckz = comp(C, w.kz);
-    const float Ax = comp(A, w.kx) - w.Sx * Akz;
-    const float Ay = comp(A, w.ky) - w.Sy * Akz;
-    const float Bx = comp(B, w.kx) - w.Sx * Bkz;
-    const float By = comp(B, w.ky) - w.Sy * Bkz;
-    const float Cx = comp(C, w.kx) - w.Sx * Ckz;
-    const float Cy = comp(C, w.ky) - w.Sy * Ckz;
+    const float Akz = vz.x - w.oz, Bkz = vz.y - w.oz, Ckz = vz.z - w.oz;
+    const float Ax = (vx.x - w.ox) - w.Sx * Akz;
+    const float Ay = (vy.x - w.oy) - w.Sy * Akz;
+    const float Bx = (vx.y - w.ox) - w.Sx * Bkz;
+    const float By = (vy.y - w.oy) - w.Sy * Bkz;
+    const float Cx = (vx.z - w.ox) - w.Sx * Ckz;
+    const float Cy = (vy.z - w.oy) - w.Sy * Ckz;
     const float U = Cx * By - Cy * Bx;
     const float V = Ax * Cy - Ay * Cx;
     const float W = Bx * Ay - By * Ax;

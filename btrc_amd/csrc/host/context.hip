@@ -21,12 +21,15 @@ using namespace btrc;
 
 // Scratch of btrc_hip_trace_closest_noalloc, for callers that cannot
 // allocate: the batch's ray counters in the first NOALLOC_COUNTER_BYTES, then the
-// traversal's per-lane stack entries beyond the LDS part (codes, then entry
-// distances, each [entry][lane]). Every GPU the library runs on holds one
+// traversal's per-lane stack entries beyond the LDS part ([entry][lane]). Every GPU the library runs on holds one
 // copy until the process ends. Host code never uses the array's name as an
 // address: it resolves the device address once per device
 // (hipGetSymbolAddress, at context creation) and uses that.
-constexpr size_t NOALLOC_SCRATCH_BYTES = (size_t)8 << 20;
+// 64 MiB holds the entries of 16 wavefronts per CU for a tree that needs 43 (a
+// million triangles); 8 MiB held 2 (1M incoherent rays: 2.27 ms, now 0.44).
+// Trees whose one wavefront needs more than NOALLOC_WAVE_BYTES are refused.
+constexpr size_t NOALLOC_SCRATCH_BYTES = (size_t)64 << 20;
+constexpr size_t NOALLOC_WAVE_BYTES = ((size_t)8 << 20) - 2048;
 constexpr size_t NOALLOC_COUNTER_BYTES = FETCH_WORDS * sizeof(uint32_t);
 static __device__ __align__(256) unsigned char scratch[NOALLOC_SCRATCH_BYTES];
 
@@ -250,7 +253,7 @@ struct btrc_ctx
     // scene
     bool has_scene = false;
     DevBuf<BvhNode4> nodes;
-    DevBuf<float4> tris;
+    DevBuf<TraceTri> tris;
     DevBuf<TraceInstance> trace_inst;
     bool two_level = false;
     DevBuf<InstanceRec> instances;
@@ -361,8 +364,7 @@ struct btrc_ctx
     } nrc;
 
     // traversal: per-lane stack overflow and the batch fetch counter
-    DevBuf<uint32_t> ovf_code;
-    DevBuf<float> ovf_t;
+    DevBuf<uint2> ovf;
     int32_t trace_grid = 0;
     DevBuf<uint32_t> fetch;
     btrc_tuning tuning{ 0, 0, TRACE_WAVES_PER_CU, 1, 0, 0, 0, 0 };
@@ -400,9 +402,9 @@ struct btrc_ctx
         const bool postpone = (any ? tuning.any_postpone_leaves : tuning.closest_postpone_leaves) != 0;
         return postpone ? SCHED_POSTPONE : SCHED_EAGER;
     }
-    TraceOverflow trace_overflow() const
+    TraceOverflow trace_overflow(bool shadow = false) const
     {
-        return TraceOverflow{ ovf_code.ptr, ovf_t.ptr, trace_grid * TRACE_BLOCK };
+        return TraceOverflow{ ovf.ptr + (shadow ? ovf.count / 2 : 0), trace_grid * TRACE_BLOCK };
     }
     SceneView scene_view() const
     {
@@ -617,10 +619,12 @@ void set_filter(btrc_ctx *ctx, const btrc_filter_desc *f)
 // persistent traversal grid and the per-lane stack overflow it needs
 void size_traversal(btrc_ctx *ctx)
 {
-    ctx->trace_grid = ctx->cu_count * ctx->tuning.trace_waves_per_cu;
-    const size_t deep = ctx->stack_size > SHORT_STACK ? (size_t)(ctx->stack_size - SHORT_STACK) : 0;
-    ctx->ovf_code.alloc(std::max<size_t>(1, deep * ctx->trace_grid * TRACE_BLOCK));
-    ctx->ovf_t.alloc(std::max<size_t>(1, deep * ctx->trace_grid * TRACE_BLOCK));
+    const int waves = ctx->tuning.trace_waves_per_cu;
+    ctx->trace_grid = ctx->cu_count * (ctx->two_level ? std::min(waves, TRACE_WAVES_TWO_LEVEL) : waves);
+    const size_t deep = ctx->stack_size > SHORT_STACK_MIN ? (size_t)(ctx->stack_size - SHORT_STACK_MIN) : 0;
+    // two areas: a bounce's shadow rays are traced beside the next bounce's
+    // extension rays
+    ctx->ovf.alloc(std::max<size_t>(1, 2 * deep * ctx->trace_grid * TRACE_BLOCK));
     ctx->fetch.alloc(FETCH_WORDS);
 }
 
@@ -628,7 +632,7 @@ void size_traversal(btrc_ctx *ctx)
 struct Accel
 {
     std::vector<BvhNode4> nodes;     // child slots hold traversal codes
-    std::vector<float4> tris;        // 3 per triangle in leaf order
+    std::vector<TraceTri> tris;      // leaf order
     std::vector<TraceInstance> inst; // two levels only
     bool on_device = false;          // built on the GPU straight into the context's buffers
     int64_t device_nodes = 0;
@@ -674,14 +678,11 @@ Accel build_flat(const std::vector<float> &world, const std::vector<uint32_t> &t
     opt.max_leaf_size = 4; // leaf codes carry counts 1..4
     const Bvh4 bvh = build_bvh4(world.data(), ntri, opt);
     Accel acc;
-    acc.tris.resize(3 * (size_t)ntri);
+    acc.tris.resize(ntri);
     for(uint32_t k = 0; k < ntri; ++k)
     {
         const uint32_t gid = bvh.prim_order[k];
-        const float *w = world.data() + 9 * (size_t)gid;
-        acc.tris[3 * k + 0] = make_float4(w[0], w[1], w[2], u2f(gid));
-        acc.tris[3 * k + 1] = make_float4(w[3], w[4], w[5], u2f(tri_inst[gid]));
-        acc.tris[3 * k + 2] = make_float4(w[6], w[7], w[8], u2f(tri_prim[gid]));
+        acc.tris[k] = make_trace_tri(world.data() + 9 * (size_t)gid, gid, tri_inst[gid], tri_prim[gid]);
     }
     append_nodes(acc, bvh, 0);
     acc.depth = bvh.depth;
@@ -732,7 +733,7 @@ Accel build_flat_gpu(btrc_ctx *ctx, const std::vector<float> &world, const std::
     ctx->nodes.alloc(b4.node_count);
     BTRC_HIP_CHECK(hipMemcpyAsync(ctx->nodes.ptr, ctx->ploc.nodes4, b4.node_count * sizeof(BvhNode4),
                                   hipMemcpyDeviceToDevice, s));
-    ctx->tris.alloc(3 * (size_t)ntri);
+    ctx->tris.alloc(ntri);
     gather_triangles(dv.ptr, dinst.ptr, dprim.ptr, ctx->ploc.prims, ntri, ctx->tris.ptr, s);
     BTRC_HIP_CHECK(hipGetLastError());
     BTRC_HIP_CHECK(hipStreamSynchronize(s));
@@ -858,16 +859,13 @@ Accel build_two_level(const btrc_scene_desc *sd, const std::vector<InstanceRec> 
         const btrc_geometry_desc &g = sd->geometries[gi];
         const uint32_t n = (uint32_t)g.triangle_count;
         const Bvh4 blas = build_bvh4(g.positions, n, bopt);
-        const uint32_t tri_base = (uint32_t)(acc.tris.size() / 3);
+        const uint32_t tri_base = (uint32_t)acc.tris.size();
         groot[gi] = (uint32_t)acc.nodes.size();
         append_nodes(acc, blas, tri_base);
         for(uint32_t k = 0; k < n; ++k)
         {
             const uint32_t prim = blas.prim_order[k];
-            const float *p = g.positions + 9 * (size_t)prim;
-            acc.tris.push_back(make_float4(p[0], p[1], p[2], u2f(prim)));
-            acc.tris.push_back(make_float4(p[3], p[4], p[5], 0.0f));
-            acc.tris.push_back(make_float4(p[6], p[7], p[8], 0.0f));
+            acc.tris.push_back(make_trace_tri(g.positions + 9 * (size_t)prim, prim, 0, prim));
         }
         blas_stack = std::max(blas_stack, blas.stack_bound);
         blas_depth = std::max(blas_depth, blas.depth);
@@ -1974,7 +1972,8 @@ void render(btrc_ctx *ctx, const btrc_render_params *p, int32_t view_count, cons
                   nrc_on ? ctx->sh_train.ptr : nullptr, nrc_on ? ctx->nrc.acc[ctx->nrc.set].ptr : nullptr };
 
     const int grid256 = ctx->persistent_grid(256, (int64_t)P);
-    const TraceOverflow ovf = ctx->trace_overflow();
+    const int shadow_grid = std::min(ctx->trace_grid, ctx->cu_count * (media ? TRACE_WAVES_MEDIA : TRACE_WAVES_ANY));
+    const TraceOverflow ovf = ctx->trace_overflow(), shadow_ovf = ctx->trace_overflow(true);
 
     // the constants live in device memory so that a captured loop stays
     // valid from one render to the next
@@ -2030,13 +2029,13 @@ void render(btrc_ctx *ctx, const btrc_render_params *p, int32_t view_count, cons
         {
             BTRC_HIP_CHECK(hipEventRecord(ctx->shaded, s));
             BTRC_HIP_CHECK(hipStreamWaitEvent(ctx->shadow_stream, ctx->shaded, 0));
-            launch_shadow(ctx->shadow_stream, ctx->trace_grid, ctx->trace_sched(true), media, ts, sv, ctx->wc(), sh,
-                          fv, ovf, side);
+            launch_shadow(ctx->shadow_stream, shadow_grid, ctx->trace_sched(true), media, ts, sv, ctx->wc(), sh,
+                          fv, shadow_ovf, side);
             BTRC_HIP_CHECK(hipEventRecord(ctx->shadow_done, ctx->shadow_stream));
             shadow_open = true;
         }
         else
-            run(STAGE_SHADOW, [&] { launch_shadow(s, ctx->trace_grid, ctx->trace_sched(true), media, ts, sv, ctx->wc(), sh, fv, ovf, side); });
+            run(STAGE_SHADOW, [&] { launch_shadow(s, shadow_grid, ctx->trace_sched(true), media, ts, sv, ctx->wc(), sh, fv, shadow_ovf, side); });
         launch_end_iteration(s, ctx->wc(), side);
     };
 
@@ -2050,7 +2049,7 @@ void render(btrc_ctx *ctx, const btrc_render_params *p, int32_t view_count, cons
             key.insert(key.end(), b, b + sizeof(v));
         };
         add(ts); add(sv); add(hit); add(sh); add(fv); add(nv); add(rcd);
-        add(ovf.code); add(ovf.t); add(ovf.lanes);
+        add(ovf.entry); add(ovf.lanes); add(shadow_ovf.entry);
         add(ctx->pool[0].view()); add(ctx->pool[1].view()); add(ctx->wc());
         // the shadow stream pays off once a bounce fills the GPU: the event
         // hand-offs cost ~6 us per bounce (256^2 frames: +8 %), the overlap
@@ -2146,7 +2145,7 @@ void render(btrc_ctx *ctx, const btrc_render_params *p, int32_t view_count, cons
                               path, hit, ctx->medium_scatter.ptr, next, sh, fv, cur);
             });
         timer.run(STAGE_SHADE, [&] { launch_shade(s, grid256, p->sampler, rcd, sv, ctx->wc(), path, hit, next, sh, fv, nv, cur); });
-        timer.run(STAGE_SHADOW, [&] { launch_shadow(s, ctx->trace_grid, ctx->trace_sched(true), media, ts, sv, ctx->wc(), sh, fv, ovf, cur); });
+        timer.run(STAGE_SHADOW, [&] { launch_shadow(s, shadow_grid, ctx->trace_sched(true), media, ts, sv, ctx->wc(), sh, fv, shadow_ovf, cur); });
         launch_end_iteration(s, ctx->wc(), cur);
         BTRC_HIP_CHECK(hipGetLastError());
         cur ^= 1;
@@ -2308,7 +2307,9 @@ void check_batch_args(btrc_ctx *ctx, const void *rays, int64_t n, int32_t tri_te
 void trace_batch(btrc_ctx *ctx, int32_t tri_test, bool any_hit, const float4 *rays, int64_t n, uint32_t *out)
 {
     BTRC_HIP_CHECK(hipMemsetAsync(ctx->fetch.ptr, 0, FETCH_WORDS * sizeof(uint32_t), ctx->stream));
-    launch_trace_batch(ctx->stream, ctx->trace_grid, ctx->trace_sched(any_hit != 0), ctx->trace_scene(), tri_test, any_hit, rays,
+    const int most = any_hit ? std::min(ctx->trace_grid, ctx->cu_count * TRACE_WAVES_ANY) : ctx->trace_grid;
+    const int grid = (int)std::max<int64_t>(1, std::min<int64_t>(most, (n + TRACE_BLOCK - 1) / TRACE_BLOCK));
+    launch_trace_batch(ctx->stream, grid, ctx->trace_sched(any_hit != 0), ctx->trace_scene(), tri_test, any_hit, rays,
                        (int32_t)n, out, ctx->fetch.ptr, ctx->trace_overflow());
     BTRC_HIP_CHECK(hipGetLastError());
 }
@@ -2891,26 +2892,25 @@ int btrc_hip_trace_closest_noalloc(btrc_ctx *ctx, const btrc_ray *rays, int64_t 
         check_range(rays, (size_t)n * sizeof(btrc_ray), "rays");
         check_range(hits, (size_t)n * sizeof(btrc_hit), "hits");
         // the persistent grid, capped so that its stack entries fit the scratch
-        const size_t deep = ctx->stack_size > SHORT_STACK ? (size_t)(ctx->stack_size - SHORT_STACK) : 0;
-        const size_t per_wave = deep * TRACE_BLOCK * (sizeof(uint32_t) + sizeof(float));
+        const size_t deep = ctx->stack_size > SHORT_STACK_MIN ? (size_t)(ctx->stack_size - SHORT_STACK_MIN) : 0;
+        const size_t per_wave = deep * TRACE_BLOCK * sizeof(uint2);
         const size_t room = NOALLOC_SCRATCH_BYTES - NOALLOC_COUNTER_BYTES;
         int waves = ctx->trace_grid;
         if(per_wave > 0 && (size_t)waves * per_wave > room)
             waves = (int)(room / per_wave);
-        if(waves < 1)
+        if(per_wave > NOALLOC_WAVE_BYTES || waves < 1)
             throw InvalidArg("scene tree too deep for the no-allocation scratch: " + std::to_string(ctx->stack_size) +
                              " stack entries need " + std::to_string(per_wave) + " bytes per wavefront beyond the " +
-                             std::to_string(room) + " the scratch holds");
+                             std::to_string(NOALLOC_WAVE_BYTES) + " the scratch allows");
         uint8_t *base = static_cast<uint8_t *>(ctx->noalloc_scratch);
         uint32_t *fetch = reinterpret_cast<uint32_t *>(base);
         const size_t lanes = (size_t)waves * TRACE_BLOCK;
-        uint32_t *ovf_code = reinterpret_cast<uint32_t *>(base + NOALLOC_COUNTER_BYTES);
-        float *ovf_t = reinterpret_cast<float *>(base + NOALLOC_COUNTER_BYTES + deep * lanes * sizeof(uint32_t));
+        uint2 *entry = reinterpret_cast<uint2 *>(base + NOALLOC_COUNTER_BYTES);
         launch_fill_u32(ctx->stream, fetch, FETCH_WORDS, 0u);
         BTRC_HIP_CHECK(hipGetLastError());
         launch_trace_batch(ctx->stream, waves, ctx->trace_sched(false), ctx->trace_scene(), tri_test, false,
                            reinterpret_cast<const float4 *>(rays), (int32_t)n, reinterpret_cast<uint32_t *>(hits),
-                           fetch, TraceOverflow{ ovf_code, ovf_t, (int32_t)lanes });
+                           fetch, TraceOverflow{ entry, (int32_t)lanes });
         BTRC_HIP_CHECK(hipGetLastError());
         BTRC_HIP_CHECK(hipStreamSynchronize(ctx->stream));
     });

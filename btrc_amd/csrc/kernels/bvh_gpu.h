@@ -17,6 +17,7 @@
 #include <vector>
 
 #include "../core/traverse.h"
+#include "trace.h"
 
 namespace btrc {
 
@@ -96,12 +97,12 @@ Bvh4Device ploc_to_bvh4(PlocBuffers &buf, const PlocResult &r, hipStream_t s);
 // what it holds (a leaf's triangles from the leaf-ordered records, an inner
 // slot's child node), level by level from the deepest; `order` lists the
 // nodes grouped by level, `levels` the group boundaries (root level first).
-void refit_bvh4(BvhNode4 *nodes, const uint32_t *order, const std::vector<uint32_t> &levels, const float4 *tris,
+void refit_bvh4(BvhNode4 *nodes, const uint32_t *order, const std::vector<uint32_t> &levels, const TraceTri *tris,
                 hipStream_t s);
 
 // The leaf-ordered triangle records of a one-level structure:
 // (v0, flattened index), (v1, instance), (v2, primitive) per leaf slot.
 void gather_triangles(const float *vertices, const uint32_t *tri_inst, const uint32_t *tri_prim,
-                      const uint32_t *prims, uint32_t n, float4 *tris, hipStream_t s);
+                      const uint32_t *prims, uint32_t n, TraceTri *tris, hipStream_t s);
 
 } // namespace btrc

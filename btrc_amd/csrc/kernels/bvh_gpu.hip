@@ -530,7 +530,7 @@ __global__ void k_bvh4_write(const PlocNode *nodes, const uint32_t *frontier, ui
 }
 
 // one level of refit_bvh4
-__global__ void k_refit4(BvhNode4 *nodes, const uint32_t *order, uint32_t lo, uint32_t hi, const float4 *tris)
+__global__ void k_refit4(BvhNode4 *nodes, const uint32_t *order, uint32_t lo, uint32_t hi, const TraceTri *tris)
 {
     const uint32_t k = lo + blockIdx.x * blockDim.x + threadIdx.x;
     if(k >= hi)
@@ -545,12 +545,13 @@ __global__ void k_refit4(BvhNode4 *nodes, const uint32_t *order, uint32_t lo, ui
         if(code & CODE_LEAF)
         {
             const uint32_t first = code & 0x0fffffffu, count = ((code >> 28) & 3u) + 1;
-            for(uint32_t t = 0; t < 3 * count; ++t)
-            {
-                const float4 v = tris[3 * (size_t)first + t];
-                b[0] = fminf(b[0], v.x); b[1] = fminf(b[1], v.y); b[2] = fminf(b[2], v.z);
-                b[3] = fmaxf(b[3], v.x); b[4] = fmaxf(b[4], v.y); b[5] = fmaxf(b[5], v.z);
-            }
+            for(uint32_t t = 0; t < count; ++t)
+                for(int a = 0; a < 3; ++a)
+                {
+                    const float4 v = *reinterpret_cast<const float4 *>(tris[(size_t)first + t].v[a]);
+                    b[a] = fminf(fminf(fminf(b[a], v.x), v.y), v.z);
+                    b[3 + a] = fmaxf(fmaxf(fmaxf(b[3 + a], v.x), v.y), v.z);
+                }
         }
         else
         {
@@ -567,16 +568,13 @@ __global__ void k_refit4(BvhNode4 *nodes, const uint32_t *order, uint32_t lo, ui
 }
 
 __global__ void k_gather_tris(const float *v, const uint32_t *tri_inst, const uint32_t *tri_prim, const uint32_t *prims,
-                              uint32_t n, float4 *tris)
+                              uint32_t n, TraceTri *tris)
 {
     const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
     if(k >= n)
         return;
     const uint32_t gid = prims[k];
-    const float *w = v + 9 * (size_t)gid;
-    tris[3 * (size_t)k + 0] = make_float4(w[0], w[1], w[2], __uint_as_float(gid));
-    tris[3 * (size_t)k + 1] = make_float4(w[3], w[4], w[5], __uint_as_float(tri_inst[gid]));
-    tris[3 * (size_t)k + 2] = make_float4(w[6], w[7], w[8], __uint_as_float(tri_prim[gid]));
+    tris[k] = make_trace_tri(v + 9 * (size_t)gid, gid, tri_inst[gid], tri_prim[gid]);
 }
 
 // the first frontier: binary root, 4-wide node 0, nothing pushed above it
@@ -867,7 +865,7 @@ Bvh4Device ploc_to_bvh4(PlocBuffers &buf, const PlocResult &r, hipStream_t s)
     return out;
 }
 
-void refit_bvh4(BvhNode4 *nodes, const uint32_t *order, const std::vector<uint32_t> &levels, const float4 *tris,
+void refit_bvh4(BvhNode4 *nodes, const uint32_t *order, const std::vector<uint32_t> &levels, const TraceTri *tris,
                 hipStream_t s)
 {
     for(size_t d = levels.size() - 1; d-- > 0;)
@@ -880,7 +878,7 @@ void refit_bvh4(BvhNode4 *nodes, const uint32_t *order, const std::vector<uint32
 }
 
 void gather_triangles(const float *vertices, const uint32_t *tri_inst, const uint32_t *tri_prim,
-                      const uint32_t *prims, uint32_t n, float4 *tris, hipStream_t s)
+                      const uint32_t *prims, uint32_t n, TraceTri *tris, hipStream_t s)
 {
     if(n)
         hipLaunchKernelGGL(k_gather_tris, grid_for(n), dim3(BLOCK), 0, s, vertices, tri_inst, tri_prim, prims, n, tris);

@@ -281,7 +281,7 @@ void launch_halton_eval(hipStream_t s, const HaltonConsts &hc, const HaltonTable
                         const int32_t *sample_index, int32_t n, int32_t dims, float *out);
 // one-level structures: world-space triangle records of `geometry`'s
 // instances from its new local positions (9 floats per triangle)
-void launch_update_world_tris(hipStream_t s, float4 *tris, uint32_t n, const InstanceRec *insts, int32_t geometry,
+void launch_update_world_tris(hipStream_t s, TraceTri *tris, uint32_t n, const InstanceRec *insts, int32_t geometry,
                               const float *positions);
 // EnvirLightSampler::preprocess's table kernel: lum and area per tile (w * h each)
 void launch_envir_table(hipStream_t s, const TextureView &tv, int32_t tex, int32_t w, int32_t h, int32_t n_samples,

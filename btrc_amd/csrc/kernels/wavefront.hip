@@ -355,7 +355,7 @@ struct ExtensionSink
     }
     __device__ __forceinline__ void store(uint32_t i, const HitRecord &h) const
     {
-        if(h.gid != 0xffffffffu)
+        if(h.hit)
         {
             hit.flag[i] = PATH_FLAG_HAS_INTERSECTION | h.inst;
             hit.tuv[i] = make_float4(h.t, h.b1, h.b2, __uint_as_float(h.prim));
@@ -365,8 +365,15 @@ struct ExtensionSink
     }
 };
 
+// wavefronts per SIMD the traversal kernels are compiled for: what fits a CU
+// (trace.h) over its four SIMDs
+#define TRACE_WAVES(SCHED, MEDIA, ANY)                                                                         \
+    __attribute__((amdgpu_waves_per_eu(((MEDIA) ? TRACE_WAVES_MEDIA                                            \
+                                        : ((SCHED) & SCHED_TWO_LEVEL) ? TRACE_WAVES_TWO_LEVEL                  \
+                                        : (ANY) ? TRACE_WAVES_ANY : TRACE_WAVES_PER_CU) / 4)))
+
 template<int SCHED>
-__global__ void __launch_bounds__(TRACE_BLOCK) k_trace_extension(
+__global__ void __launch_bounds__(TRACE_BLOCK) TRACE_WAVES(SCHED, false, false) k_trace_extension(
     TraceScene ts, WaveCounters *c, PathSOA path, HitSOA hit, TraceOverflow ovf)
 {
     QueueState *q = queue_state(c);
@@ -1054,7 +1061,7 @@ struct ShadowSink
     }
     __device__ __forceinline__ void store(uint32_t i, const HitRecord &h) const
     {
-        if(h.gid == 0xffffffffu)
+        if(!h.hit)
         {
             const float4 a = shadow.o[i];
             const float4 b = shadow.beta[i];
@@ -1097,7 +1104,7 @@ struct ShadowSink
 };
 
 template<int SCHED, bool MEDIA>
-__global__ void __launch_bounds__(TRACE_BLOCK) k_shadow(
+__global__ void __launch_bounds__(TRACE_BLOCK) TRACE_WAVES(SCHED, MEDIA, true) k_shadow(
     TraceScene ts, SceneView sv, WaveCounters *c, ShadowSOA shadow, FilmView film, TraceOverflow ovf, int parity)
 {
     QueueState *q = queue_state(c);
@@ -1169,14 +1176,13 @@ struct BatchSink
     __device__ __forceinline__ void store(uint32_t i, const HitRecord &h) const
     {
         if(ANY)
-            out[i] = h.gid != 0xffffffffu ? 1u : 0u;
+            out[i] = h.hit ? 1u : 0u;
         else
         {
             uint32_t *o = out + 5 * (size_t)i;
-            const bool hitp = h.gid != 0xffffffffu;
             o[0] = __float_as_uint(h.t);
-            o[1] = hitp ? h.inst : 0xffffffffu;
-            o[2] = hitp ? h.prim : 0xffffffffu;
+            o[1] = h.inst;
+            o[2] = h.prim;
             o[3] = __float_as_uint(h.b1);
             o[4] = __float_as_uint(h.b2);
         }
@@ -1184,7 +1190,7 @@ struct BatchSink
 };
 
 template<int TRI, bool ANY, int SCHED>
-__global__ void __launch_bounds__(TRACE_BLOCK) k_trace_batch(
+__global__ void __launch_bounds__(TRACE_BLOCK) TRACE_WAVES(SCHED, false, ANY) k_trace_batch(
     TraceScene ts, const float4 *rays, int32_t n, uint32_t *out, uint32_t *fetch, TraceOverflow ovf)
 {
     BatchSink<ANY> sink{ rays, out };
@@ -1215,21 +1221,22 @@ __global__ void k_volume_eval(VolumeView vv, const float4 *seg, const uint2 *see
 // world-space records of a one-level structure after a geometry's vertices
 // changed: the records of every instance of `geometry` take the new
 // positions through the instance's transform, as the upload computes them
-__global__ void k_update_world_tris(float4 *tris, uint32_t n, const InstanceRec *insts, int32_t geometry,
+__global__ void k_update_world_tris(TraceTri *tris, uint32_t n, const InstanceRec *insts, int32_t geometry,
                                     const float *positions)
 {
     const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
     if(k >= n)
         return;
-    const uint32_t inst = __float_as_uint(tris[3 * (size_t)k + 1].w);
-    const InstanceRec &r = insts[inst];
+    const InstanceRec &r = insts[tris[k].inst];
     if(r.geometry_id != geometry)
         return;
-    const float *p = positions + 9 * (size_t)__float_as_uint(tris[3 * (size_t)k + 2].w);
+    const float *p = positions + 9 * (size_t)tris[k].prim;
     for(int v = 0; v < 3; ++v)
     {
         const V3 w = xf_point(r.xf, v3(p[3 * v], p[3 * v + 1], p[3 * v + 2]));
-        tris[3 * (size_t)k + v] = make_float4(w.x, w.y, w.z, tris[3 * (size_t)k + v].w);
+        tris[k].v[0][v] = w.x;
+        tris[k].v[1][v] = w.y;
+        tris[k].v[2][v] = w.z;
     }
 }
 
@@ -1550,7 +1557,7 @@ void launch_volume_eval(hipStream_t s, const VolumeView &vv, const float4 *seg, 
     hipLaunchKernelGGL(k_volume_eval, dim3((n + 127) / 128), dim3(128), 0, s, vv, seg, seed, n, out);
 }
 
-void launch_update_world_tris(hipStream_t s, float4 *tris, uint32_t n, const InstanceRec *insts, int32_t geometry,
+void launch_update_world_tris(hipStream_t s, TraceTri *tris, uint32_t n, const InstanceRec *insts, int32_t geometry,
                               const float *positions)
 {
     if(n)

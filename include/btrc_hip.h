@@ -365,7 +365,7 @@ typedef struct btrc_tuning
 {
     int32_t closest_postpone_leaves; /* one-level scenes, 1: leaves wait until every lane holds one (default 0) */
     int32_t any_postpone_leaves;     /* same for visibility rays (default 0) */
-    int32_t trace_waves_per_cu;      /* persistent traversal grid, 1..32 (default 20) */
+    int32_t trace_waves_per_cu;      /* persistent traversal grid, 1..32 (default 24; two-level scenes: at most 20) */
     int32_t launch_graph;            /* 1: the bounce loop replays a captured HIP graph (default 1) */
     int32_t two_level_postpone;      /* two-level scenes: bit 0 closest-hit, bit 1 visibility rays
                                         postpone leaves (default 0: both test leaves when reached) */
@@ -490,7 +490,7 @@ int btrc_hip_trace_any(btrc_ctx *ctx, const btrc_ray *rays, int64_t n, int32_t t
  * live in device memory (`rays` and `hits` are device or managed
  * allocations holding n entries each). It allocates nothing: the
  * traversal's ray counter and its per-lane stack entries beyond the LDS part
- * live in a static 8 MiB device array per GPU, which caps the persistent
+ * live in a static 64 MiB device array per GPU, which caps the persistent
  * grid and fails with BTRC_ERR_INVALID when the scene's tree needs more
  * stack than the array holds. Calls that overlap on one GPU race, since they
  * share that array. Returns once the hits are written. */
