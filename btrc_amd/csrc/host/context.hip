@@ -324,6 +324,7 @@ struct btrc_ctx
     // first-digit tables of the Halton sampler (built on first use)
     DevBuf<uint16_t> halton_values;
     DevBuf<HaltonDim> halton_dims;
+    DevBuf<float> sample_rows;        // the frame's Halton numbers (k_sample_rows)
 
     // film filter
     FilterConsts filter{ FILTER_BOX, 0.0f, 0.0f, nullptr };
@@ -1789,6 +1790,54 @@ std::vector<ViewRec> make_views(btrc_ctx *ctx, const btrc_render_params *p, int3
     return out;
 }
 
+// Whether a frame reads its Halton numbers from sample rows, and how many
+// samples and dimensions its rows hold (samples 0: the stages run the digit
+// loop). Rows pay off once enough pixels share each: ROWS_MIN_SHARE. They
+// hold every dimension a path can draw: four for the camera, eight per vertex,
+// the last one at the larger of the two depths (all 998 with media, whose tracking steps draw without a bound). Frames of
+// more samples than ROWS_MAX_BYTES holds go through in windows of samples,
+// which needs sample-major paths: one view in uniform order.
+constexpr uint64_t ROWS_MIN_SHARE = 12;
+constexpr size_t ROWS_MAX_BYTES = (size_t)2 << 30;
+
+struct SampleRows
+{
+    int32_t samples = 0, dims = 0;
+};
+
+SampleRows plan_sample_rows(btrc_ctx *ctx, const btrc_render_params *p, const std::vector<ViewRec> &views,
+                            uint64_t pixels, bool media)
+{
+    SampleRows r;
+    if(p->sampler != BTRC_SAMPLER_HALTON || pixels < ROWS_MIN_SHARE * (uint64_t)ROW_CELLS)
+        return r;
+    for(const ViewRec &v : views)
+        if(v.width < MAX_HALTON_RESOLUTION || v.height < MAX_HALTON_RESOLUTION)
+            return r; // another stride, other indices
+    const int64_t most = PRIME_TABLE_SIZE - 2;
+    const int64_t need = media ? most : std::min<int64_t>(most, 4 + 8 * ((int64_t)std::max(p->min_depth, p->max_depth) + 1));
+    const int64_t dims = (need + 3) / 4 * 4;
+    const int64_t fit = (int64_t)(ROWS_MAX_BYTES / ((size_t)ROW_CELLS * dims * sizeof(float)));
+    if(p->spp > fit && (views.size() > 1 || p->tile))
+        return r;
+    r.samples = (int32_t)std::min<int64_t>(p->spp, fit);
+    r.dims = (int32_t)dims;
+    const size_t floats = (size_t)r.samples * ROW_CELLS * dims;
+    if(ctx->sample_rows.count < floats)
+    {
+        try
+        {
+            ctx->sample_rows.alloc(floats);
+        }
+        catch(const std::bad_alloc &)
+        {
+            (void)hipGetLastError(); // no room: the digit loop needs none
+            return SampleRows();
+        }
+    }
+    return r;
+}
+
 void render(btrc_ctx *ctx, const btrc_render_params *p, int32_t view_count, const btrc_view_desc *view_desc,
             btrc_render_stats *stats, int32_t capture_bounces, btrc_ray *capture, int64_t capture_max,
             int64_t *capture_count)
@@ -1898,16 +1947,14 @@ void render(btrc_ctx *ctx, const btrc_render_params *p, int32_t view_count, cons
             if(r.complete_stage)
                 r.complete_stage(r.user);
         }
-        void progress(const WaveCounters &c) const
+        void progress(const WaveCounters &c, uint64_t total) const
         {
-            if(r.progress && c.total > 0)
-                r.progress(r.user, (float)(100.0 * (double)(c.generated - (uint64_t)c.active) / (double)c.total));
+            if(r.progress && total > 0)
+                r.progress(r.user, (float)(100.0 * (double)(c.generated - (uint64_t)c.active) / (double)total));
         }
     } reporter_stage(ctx->reporter);
 
-    WaveCounters init{};
-    init.total = total;
-    *ctx->host_counters = init;
+    *ctx->host_counters = WaveCounters{};
     BTRC_HIP_CHECK(hipMemsetAsync(ctx->counters.ptr, 0, sizeof(WaveState), s));
     BTRC_HIP_CHECK(hipMemcpyAsync(ctx->wc(), ctx->host_counters, sizeof(WaveCounters), hipMemcpyHostToDevice, s));
 
@@ -1948,6 +1995,10 @@ void render(btrc_ctx *ctx, const btrc_render_params *p, int32_t view_count, cons
     }
     rc.filter = ctx->filter;
     rc.halton = halton_tables(ctx);
+    const SampleRows rows = plan_sample_rows(ctx, p, views, pixels, media);
+    const int sampler = rows.samples > 0 ? (int)SAMPLER_HALTON_ROWS : (int)p->sampler;
+    rc.rows = rows.samples > 0 ? ctx->sample_rows.ptr : nullptr;
+    rc.row_dims = rows.dims;
 
     const TraceScene ts = ctx->trace_scene();
     SceneView sv = ctx->scene_view();
@@ -1980,9 +2031,31 @@ void render(btrc_ctx *ctx, const btrc_render_params *p, int32_t view_count, cons
     if(!ctx->rc_host)
         BTRC_HIP_CHECK(hipHostMalloc((void **)&ctx->rc_host, sizeof(RenderConsts), hipHostMallocDefault));
     ctx->rc_dev.alloc(1);
-    *ctx->rc_host = rc;
-    BTRC_HIP_CHECK(hipMemcpyAsync(ctx->rc_dev.ptr, ctx->rc_host, sizeof(RenderConsts), hipMemcpyHostToDevice, s));
     const RenderConsts *rcd = ctx->rc_dev.ptr;
+    // The bounce loop runs once per window of samples: the whole frame, or as
+    // many samples as the sample rows hold. Every launch of the previous
+    // window has ended when the next one's constants and rows are written.
+    uint64_t window_total = 0;
+    int32_t window_sample = 0;
+    auto next_window = [&]() -> bool {
+        if(window_total == total)
+            return false;
+        const int32_t left = p->spp - window_sample;
+        const int32_t samples = rows.samples > 0 ? std::min(left, rows.samples) : left;
+        rc.row_sample = p->sample_offset + window_sample;
+        window_sample += samples;
+        // several windows: one view, samples in the outer order
+        window_total = window_sample == p->spp ? total : (uint64_t)pixels * (uint64_t)window_sample;
+        rc.total = window_total;
+        *ctx->rc_host = rc;
+        BTRC_HIP_CHECK(hipMemcpyAsync(ctx->rc_dev.ptr, ctx->rc_host, sizeof(RenderConsts), hipMemcpyHostToDevice, s));
+        if(rows.samples > 0)
+        {
+            launch_sample_rows(s, views[0].halton, rc.halton, rc.row_sample, samples, rows.dims, ctx->sample_rows.ptr);
+            BTRC_HIP_CHECK(hipGetLastError());
+        }
+        return true;
+    };
 
     StageTimer timer;
     timer.enabled = p->time_stages != 0;
@@ -2009,22 +2082,22 @@ void render(btrc_ctx *ctx, const btrc_render_params *p, int32_t view_count, cons
     auto enqueue_bounce = [&](int side, bool timed, bool overlap) {
         PathSOA path = ctx->pool[side].view();
         PathSOA next = ctx->pool[side ^ 1].view();
-        launch_plan(s, ctx->wc(), p->state_count, side);
+        launch_plan(s, rcd, ctx->wc(), p->state_count, side);
         auto run = [&](int stage, auto &&fn) {
             if(timed)
                 timer.run(stage, fn);
             else
                 fn();
         };
-        run(STAGE_GENERATE, [&] { launch_generate(s, grid256, p->sampler, rcd, ctx->wc(), path); });
+        run(STAGE_GENERATE, [&] { launch_generate(s, grid256, sampler, rcd, ctx->wc(), path); });
         run(STAGE_TRACE, [&] { launch_trace_extension(s, ctx->trace_grid, ctx->trace_sched(false), ts, ctx->wc(), path, hit, ovf); });
         join_shadow();
         if(media)
             run(STAGE_MEDIUM, [&] {
-                launch_medium(s, grid256, ctx->cu_count * MEDIUM_TRACK_WAVES_PER_CU, p->sampler, rcd, sv, ctx->wc(),
+                launch_medium(s, grid256, ctx->cu_count * MEDIUM_TRACK_WAVES_PER_CU, sampler, rcd, sv, ctx->wc(),
                               path, hit, ctx->medium_scatter.ptr, next, sh, fv, side);
             });
-        run(STAGE_SHADE, [&] { launch_shade(s, grid256, p->sampler, rcd, sv, ctx->wc(), path, hit, next, sh, fv, nv, side); });
+        run(STAGE_SHADE, [&] { launch_shade(s, grid256, sampler, rcd, sv, ctx->wc(), path, hit, next, sh, fv, nv, side); });
         if(overlap)
         {
             BTRC_HIP_CHECK(hipEventRecord(ctx->shaded, s));
@@ -2056,7 +2129,7 @@ void render(btrc_ctx *ctx, const btrc_render_params *p, int32_t view_count, cons
         // saves ~7 % of a 1080p frame
         const bool overlap = std::min<uint64_t>((uint64_t)p->state_count, total) >= (1u << 20);
         const int32_t ints[9] = { grid256, ctx->trace_grid, ctx->trace_sched(false), ctx->trace_sched(true),
-                                  p->sampler, p->state_count, media ? 1 : 0, check_every, overlap ? 1 : 0 };
+                                  sampler, p->state_count, media ? 1 : 0, check_every, overlap ? 1 : 0 };
         add(ints);
         int g = -1;
         for(int k = 0; k < 2; ++k)
@@ -2085,6 +2158,7 @@ void render(btrc_ctx *ctx, const btrc_render_params *p, int32_t view_count, cons
             }
             ctx->loop_key[g] = key;
         }
+        while(next_window())
         for(;;)
         {
             if(ctx->stop.load())
@@ -2093,20 +2167,21 @@ void render(btrc_ctx *ctx, const btrc_render_params *p, int32_t view_count, cons
             BTRC_HIP_CHECK(hipMemcpyAsync(ctx->host_counters, ctx->wc(), sizeof(WaveCounters), hipMemcpyDeviceToHost, s));
             BTRC_HIP_CHECK(hipStreamSynchronize(s));
             const WaveCounters &hc = *ctx->host_counters;
-            reporter_stage.progress(hc);
-            if(hc.generated == hc.total && hc.active == 0)
+            reporter_stage.progress(hc, total);
+            if(hc.generated == window_total && hc.active == 0)
                 break;
         }
     }
     else
-    for(uint64_t iter = 0;; ++iter)
+    for(uint64_t iter = 0; next_window();)
+    for(;; ++iter)
     {
         if(ctx->stop.load())
             throw Stopped("render stopped");
         PathSOA path = ctx->pool[cur].view();
         PathSOA next = ctx->pool[cur ^ 1].view();
-        launch_plan(s, ctx->wc(), p->state_count, cur);
-        timer.run(STAGE_GENERATE, [&] { launch_generate(s, grid256, p->sampler, rcd, ctx->wc(), path); });
+        launch_plan(s, rcd, ctx->wc(), p->state_count, cur);
+        timer.run(STAGE_GENERATE, [&] { launch_generate(s, grid256, sampler, rcd, ctx->wc(), path); });
         timer.run(STAGE_TRACE, [&] { launch_trace_extension(s, ctx->trace_grid, ctx->trace_sched(false), ts, ctx->wc(), path, hit, ovf); });
         if(capture && (int64_t)iter < capture_bounces && captured < capture_max)
         {
@@ -2141,10 +2216,10 @@ void render(btrc_ctx *ctx, const btrc_render_params *p, int32_t view_count, cons
         }
         if(media)
             timer.run(STAGE_MEDIUM, [&] {
-                launch_medium(s, grid256, ctx->cu_count * MEDIUM_TRACK_WAVES_PER_CU, p->sampler, rcd, sv, ctx->wc(),
+                launch_medium(s, grid256, ctx->cu_count * MEDIUM_TRACK_WAVES_PER_CU, sampler, rcd, sv, ctx->wc(),
                               path, hit, ctx->medium_scatter.ptr, next, sh, fv, cur);
             });
-        timer.run(STAGE_SHADE, [&] { launch_shade(s, grid256, p->sampler, rcd, sv, ctx->wc(), path, hit, next, sh, fv, nv, cur); });
+        timer.run(STAGE_SHADE, [&] { launch_shade(s, grid256, sampler, rcd, sv, ctx->wc(), path, hit, next, sh, fv, nv, cur); });
         timer.run(STAGE_SHADOW, [&] { launch_shadow(s, shadow_grid, ctx->trace_sched(true), media, ts, sv, ctx->wc(), sh, fv, shadow_ovf, cur); });
         launch_end_iteration(s, ctx->wc(), cur);
         BTRC_HIP_CHECK(hipGetLastError());
@@ -2154,9 +2229,12 @@ void render(btrc_ctx *ctx, const btrc_render_params *p, int32_t view_count, cons
             BTRC_HIP_CHECK(hipMemcpyAsync(ctx->host_counters, ctx->wc(), sizeof(WaveCounters), hipMemcpyDeviceToHost, s));
             BTRC_HIP_CHECK(hipStreamSynchronize(s));
             const WaveCounters &hc = *ctx->host_counters;
-            reporter_stage.progress(hc);
-            if(hc.generated == hc.total && hc.active == 0)
+            reporter_stage.progress(hc, total);
+            if(hc.generated == window_total && hc.active == 0)
+            {
+                ++iter;
                 break;
+            }
         }
     }
     int32_t nrc_steps = 0;

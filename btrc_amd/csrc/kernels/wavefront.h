@@ -22,7 +22,7 @@ struct PathSOA
     float4 *beta;     // throughput.xyz, depth bits
     float4 *rad;      // path radiance.xyz, training path id bits (cache mode) or ~0
     float4 *bsdf_le;  // beta_le.xyz, bsdf pdf (negative: delta lobe)
-    uint4 *smp;       // pixel index, then Halton: dimension, index, 0;
+    uint4 *smp;       // pixel index, then Halton: dimension, index, sample row;
                       // independent: PCG state lo, hi, unused
 };
 
@@ -54,7 +54,6 @@ struct WaveCounters
     int32_t gen_offset;   // dense index of the first generated state
     int32_t pad0;
     uint64_t generated;   // paths generated so far
-    uint64_t total;       // spp * width * height
     uint64_t gen_base;    // path index of the first generated state
     uint64_t ext_rays;    // extension rays traced
     uint64_t shadow_rays; // shadow rays traced
@@ -161,6 +160,8 @@ enum : int32_t
 {
     SAMPLER_HALTON = 0,
     SAMPLER_INDEPENDENT = 1,
+    // SAMPLER_HALTON's numbers read from sample rows (k_sample_rows)
+    SAMPLER_HALTON_ROWS = 2,
     FILTER_BOX = 0,
     FILTER_GAUSSIAN = 1,
 };
@@ -209,16 +210,42 @@ struct RenderConsts
     // paths with id pixel / nrc_stride while that is below nrc_max_paths
     int32_t nrc_stride, nrc_phase, nrc_max_paths;
     FilterConsts filter;
+    // sample rows of the frame (SAMPLER_HALTON_ROWS): row r holds dimensions 2,
+    // 3, ... of the Halton index of sample row_sample + r / ROW_CELLS at the
+    // pixels whose coordinates modulo 128 are r % ROW_CELLS
+    const float *rows;
+    int32_t row_dims;       // floats per row, a multiple of four
+    int32_t row_sample;
+    uint64_t total;         // paths to generate (of the frame, or to the end of the rows' samples)
     HaltonTables halton;    // dimensions and first-digit tables of the Halton sampler
 };
+
+// A Halton index depends on the pixel only through its coordinates modulo
+// MAX_HALTON_RESOLUTION, so the pixels of a large film share their numbers:
+// 126 of a 1080p film's pixels use each. Row of pixel (px, py) and sample.
+constexpr int32_t ROW_CELLS = MAX_HALTON_RESOLUTION * MAX_HALTON_RESOLUTION;
+
+__device__ __forceinline__ uint32_t sample_row(const RenderConsts &rc, uint32_t px, uint32_t py, int32_t sample)
+{
+    return (uint32_t)(sample - rc.row_sample) * (uint32_t)ROW_CELLS +
+           (py % (uint32_t)MAX_HALTON_RESOLUTION) * (uint32_t)MAX_HALTON_RESOLUTION + px % (uint32_t)MAX_HALTON_RESOLUTION;
+}
+
+// A pointer loaded from a device-memory record, known to be global: without
+// this its loads compile to flat ones, which also wait on the LDS counter
+template<class T> __device__ __forceinline__ const T *as_global(const T *p)
+{
+    return (const T *)(const __attribute__((address_space(1))) T *)p;
+}
 
 // the view holding film pixel `pixel`
 __device__ __forceinline__ const ViewRec &view_of_pixel(const RenderConsts &rc, uint32_t pixel)
 {
+    const ViewRec *views = as_global(rc.views);
     int32_t v = rc.view_count - 1;
-    while(v > 0 && pixel < rc.views[v].pixel_base)
+    while(v > 0 && pixel < views[v].pixel_base)
         --v;
-    return rc.views[v];
+    return views[v];
 }
 
 struct FilmView
@@ -249,7 +276,10 @@ enum : int
 };
 
 // parity: the bounce's parity (the pool side it reads)
-void launch_plan(hipStream_t s, WaveCounters *c, int32_t state_count, int parity);
+void launch_plan(hipStream_t s, const RenderConsts *rc, WaveCounters *c, int32_t state_count, int parity);
+// fills `samples` * ROW_CELLS sample rows from first sample `sample` on
+void launch_sample_rows(hipStream_t s, const HaltonConsts &hc, const HaltonTables &tab, int32_t sample, int32_t samples,
+                        int32_t dims, float *rows);
 void launch_generate(hipStream_t s, int grid, int sampler, const RenderConsts *rc, const WaveCounters *c,
                      PathSOA path);
 void launch_trace_extension(hipStream_t s, int grid, int sched, const TraceScene &ts, WaveCounters *c,

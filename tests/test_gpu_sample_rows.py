@@ -1,0 +1,72 @@
+"""Frames large enough to read their Halton numbers from sample rows: per
+pixel against the oracle at the smallest such film, with depths that draw the
+most (a minimum depth above the maximum included) and both filters; films that share too few pixels or are narrower than 128 keep the
+digit loop; frames in several windows of samples equal the same samples
+rendered separately, at a sample offset; tile order equals uniform order."""
+import numpy as np
+import pytest
+
+from btrc_amd import scenes
+from oracle import oracle
+
+from util import render_params
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("w,h,min_depth,max_depth,filt", [
+    (512, 384, 3, 8, "box"),          # 12 pixels a row: the first size with rows
+    (512, 383, 3, 8, "box"),          # just below
+    (2048, 128, 0, 3, "gaussian"),
+    (4096, 127, 3, 5, "box"),         # another stride: no rows
+    (640, 400, 9, 2, "gaussian"),     # nine vertices without roulette, then the end
+])
+def test_rows_match_oracle(ctx, w, h, min_depth, max_depth, filt):
+    scene, cam = scenes.cornell()
+    ctx.upload_scene(scene)
+    ctx.set_camera(cam, w, h)
+    ctx.set_filter(filt)
+    p = render_params(w, h, 1, min_depth=min_depth, max_depth=max_depth, state_count=1 << 18)
+    st = ctx.render(p)
+    got = ctx.film(w, h)[0][..., :3].astype(np.float64)
+    ctx.set_filter("box")
+    r0, r1 = h // 2, h // 2 + 24
+    ref = oracle.OracleScene(scene).render(cam, p, first=r0 * w, count=(r1 - r0) * w,
+                                           filt=None if filt == "box" else ("gaussian", 1.3, 1.6))[0][r0:r1]
+    rel = np.abs(got[r0:r1] - ref) / np.maximum(np.abs(ref), 1e-2)
+    assert rel.max() <= 1e-4 and ref.max() > 0
+    assert st.paths == w * h
+
+
+def fp64_film(ctx, w, h, spp, offset=0, accumulate=0, tile=0, state_count=1 << 20):
+    p = render_params(w, h, spp, min_depth=3, max_depth=6, state_count=state_count, film_fp64=1)
+    p.sample_offset, p.accumulate, p.tile = offset, accumulate, tile
+    st = ctx.render(p)
+    return ctx.film(w, h, fp64=True)[1], st.extension_rays
+
+
+@pytest.mark.parametrize("graph", [1, 0])
+def test_windows_of_samples(ctx, graph):
+    # media rows hold 998 dimensions: 32 samples fill the rows' memory, so 40
+    # samples take two windows
+    scene, cam = scenes.cornell_media(grid=scenes.fbm_grid(16, octaves=3, seed=3, max_sigma=0.2))
+    ctx.upload_scene(scene)
+    w, h = 512, 400
+    ctx.set_camera(cam, w, h)
+    ctx.set_tuning(launch_graph=graph)
+    whole, rays = fp64_film(ctx, w, h, 40)
+    _, first = fp64_film(ctx, w, h, 20)
+    parts, second = fp64_film(ctx, w, h, 20, offset=20, accumulate=1)
+    ctx.set_tuning(launch_graph=1)
+    assert rays == first + second
+    assert np.abs(whole - parts).max() <= 1e-12 * max(1.0, np.abs(parts).max())
+
+
+def test_tile_order_equals_uniform(ctx):
+    scene, cam = scenes.cornell()
+    ctx.upload_scene(scene)
+    ctx.set_camera(cam, 600, 400)
+    a, ra = fp64_film(ctx, 600, 400, 3)
+    b, rb = fp64_film(ctx, 600, 400, 3, tile=1, state_count=100000)
+    assert ra == rb
+    assert np.abs(a - b).max() <= 1e-12 * max(1.0, np.abs(a).max())
