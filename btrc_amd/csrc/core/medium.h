@@ -42,10 +42,11 @@ struct MediumRec
     float g;                // Henyey-Greenstein asymmetry
     int32_t nx, ny, nz;     // voxel grid, x fastest
     int32_t albedo_grid;    // 1: 3 floats per voxel at albedo_offset
-    uint32_t density_offset; // first voxel in SceneView::voxels
+    uint32_t density_offset; // first voxel in Grids::voxels
     uint32_t albedo_offset;
     float world_to_local[12]; // row-major 3x4
-    float pad[2];
+    uint32_t brick_offset;  // the density grid's first brick (Grids::bricks)
+    float pad;
 };
 
 BTRC_HD float henyey_greenstein(float g, float u)
@@ -127,6 +128,70 @@ BTRC_HD float grid_lookup(const float *g, int32_t nx, int32_t ny, int32_t nz, in
     return lerpf(c0, c1, tz);
 }
 
+// Density grids as the tracking loops read them: bricks of 3 x 3 x 3 voxels
+// (x fastest), one 128-byte line each, covering the 2 x 2 x 2 cells between
+// them; neighbouring bricks share their border voxels. All eight voxels of a
+// lookup come from one line, where the plain grid's four rows lie in four or
+// five (a step's random lookups ran into the L2's request rate: 14 TB/s of
+// lines; media frame, 1080p at 4 spp: 46.0 ms of tracking, 36.3 from bricks).
+// Four times the grid's memory.
+constexpr int32_t BRICK_FLOATS = 32;
+
+struct Grids
+{
+    const float *voxels; // plain grids: albedos, and the densities bricks are made of
+    const float *bricks; // density grids
+};
+
+// bricks along an axis of n voxels
+BTRC_HD int32_t brick_count(int32_t n) { return n < 4 ? 1 : n / 2; }
+
+// voxel of grid g in element e (below 27) of brick b
+BTRC_HD float brick_element(const float *g, int32_t nx, int32_t ny, int32_t nz, uint32_t b, uint32_t e)
+{
+    const uint32_t bx = (uint32_t)brick_count(nx), by = (uint32_t)brick_count(ny);
+    const int32_t x = (int32_t)(2 * (b % bx) + e % 3), y = (int32_t)(2 * (b / bx % by) + e / 3 % 3),
+                  z = (int32_t)(2 * (b / bx / by) + e / 9);
+    const int32_t cx = x < nx ? x : nx - 1, cy = y < ny ? y : ny - 1, cz = z < nz ? z : nz - 1;
+    return g[((size_t)cz * ny + cy) * nx + cx];
+}
+
+struct FloatPair
+{
+    float a, b;
+};
+
+// grid_lookup of a one-channel grid from its bricks: the same voxels, weights
+// and order of operations
+BTRC_HD float brick_lookup(const float *bricks, int32_t nx, int32_t ny, int32_t nz, V3 uvw)
+{
+    const float x = clamp_texel_coord(uvw.x * (float)nx - 0.5f, nx);
+    const float y = clamp_texel_coord(uvw.y * (float)ny - 0.5f, ny);
+    const float z = clamp_texel_coord(uvw.z * (float)nz - 0.5f, nz);
+    const float fx = floorf(x), fy = floorf(y), fz = floorf(z);
+    const float tx = x - fx, ty = y - fy, tz = z - fz;
+    // along an axis the two voxels are the cell's (base, base + 1), or twice
+    // the border voxel: base for a coordinate below 0, base + 1 (one voxel:
+    // base) beyond the last cell
+    const int32_t ix = (int32_t)fx, iy = (int32_t)fy, iz = (int32_t)fz;
+    const int32_t mx = nx < 2 ? 0 : nx - 2, my = ny < 2 ? 0 : ny - 2, mz = nz < 2 ? 0 : nz - 2;
+    const int32_t cx = ix < 0 ? 0 : (ix > mx ? mx : ix), cy = iy < 0 ? 0 : (iy > my ? my : iy),
+                  cz = iz < 0 ? 0 : (iz > mz ? mz : iz);
+    const bool x0 = ix > mx && nx > 1, x1 = ix >= 0 && nx > 1; // whether the lower / upper voxel is base + 1
+    const int32_t y0 = iy > my && ny > 1 ? 3 : 0, y1 = iy >= 0 && ny > 1 ? 3 : 0;
+    const int32_t z0 = iz > mz && nz > 1 ? 9 : 0, z1 = iz >= 0 && nz > 1 ? 9 : 0;
+    const uint32_t brick = ((uint32_t)(cz >> 1) * (uint32_t)brick_count(ny) + (uint32_t)(cy >> 1)) *
+                           (uint32_t)brick_count(nx) + (uint32_t)(cx >> 1);
+    const float *b = bricks + (size_t)brick * BRICK_FLOATS + ((cz & 1) * 9 + (cy & 1) * 3 + (cx & 1));
+    auto row = [&](int32_t at) {
+        FloatPair v;
+        std::memcpy(&v, b + at, sizeof(v));
+        return lerpf(x0 ? v.b : v.a, x1 ? v.b : v.a, tx);
+    };
+    const float c00 = row(y0 + z0), c10 = row(y1 + z0), c01 = row(y0 + z1), c11 = row(y1 + z1);
+    return lerpf(lerpf(c00, c10, ty), lerpf(c01, c11, ty), tz);
+}
+
 BTRC_HD V3 medium_uvw(const MediumRec &m, V3 p)
 {
     if(!m.has_xform)
@@ -178,7 +243,7 @@ BTRC_HD GridTrack grid_track_start(const MediumRec &m, V3 a, V3 b)
 // (or the step limit reached), else the grid point and its density. Smp
 // provides float get1d().
 template<class Smp>
-BTRC_HD bool grid_track_step(const MediumRec &m, const float *voxels, GridTrack &g, Smp &smp, V3 *uvw,
+BTRC_HD bool grid_track_step(const MediumRec &m, const Grids &grids, GridTrack &g, Smp &smp, V3 *uvw,
                              float *density)
 {
     if(g.it >= MAX_TRACKING_STEPS)
@@ -189,16 +254,16 @@ BTRC_HD bool grid_track_step(const MediumRec &m, const float *voxels, GridTrack 
         return false;
     ++g.it;
     *uvw = g.local_a + g.t * g.local_step;
-    *density = grid_lookup(voxels + m.density_offset, m.nx, m.ny, m.nz, 1, 0, *uvw);
+    *density = brick_lookup(grids.bricks + (size_t)m.brick_offset * BRICK_FLOATS, m.nx, m.ny, m.nz, *uvw);
     return true;
 }
 
 // the phase colour at grid point uvw
-BTRC_HD V3 grid_albedo(const MediumRec &m, const float *voxels, V3 uvw)
+BTRC_HD V3 grid_albedo(const MediumRec &m, const Grids &grids, V3 uvw)
 {
     if(!m.albedo_grid)
         return v3(m.albedo[0], m.albedo[1], m.albedo[2]);
-    const float *alb = voxels + m.albedo_offset;
+    const float *alb = grids.voxels + m.albedo_offset;
     return v3(grid_lookup(alb, m.nx, m.ny, m.nz, 3, 0, uvw), grid_lookup(alb, m.nx, m.ny, m.nz, 3, 1, uvw),
               grid_lookup(alb, m.nx, m.ny, m.nz, 3, 2, uvw));
 }
@@ -206,7 +271,7 @@ BTRC_HD V3 grid_albedo(const MediumRec &m, const float *voxels, V3 uvw)
 // Medium::sample along the segment a -> b (a, b in world space). Smp
 // provides float get1d().
 template<class Smp>
-BTRC_HD MediumSample medium_sample(const MediumRec &m, const float *voxels, V3 a, V3 b, Smp &smp)
+BTRC_HD MediumSample medium_sample(const MediumRec &m, const Grids &grids, V3 a, V3 b, Smp &smp)
 {
     MediumSample r;
     r.scattered = false;
@@ -229,13 +294,13 @@ BTRC_HD MediumSample medium_sample(const MediumRec &m, const float *voxels, V3 a
     GridTrack g = grid_track_start(m, a, b);
     V3 uvw;
     float density;
-    while(grid_track_step(m, voxels, g, smp, &uvw, &density))
+    while(grid_track_step(m, grids, g, smp, &uvw, &density))
     {
         if(smp.get1d() < density * m.inv_max_density)
         {
             r.scattered = true;
             r.position = g.a + g.t * g.world_step;
-            r.color = grid_albedo(m, voxels, uvw);
+            r.color = grid_albedo(m, grids, uvw);
             break;
         }
     }
@@ -244,7 +309,7 @@ BTRC_HD MediumSample medium_sample(const MediumRec &m, const float *voxels, V3 a
 
 // Medium::tr along a -> b
 template<class Smp>
-BTRC_HD V3 medium_tr(const MediumRec &m, const float *voxels, V3 a, V3 b, Smp &smp)
+BTRC_HD V3 medium_tr(const MediumRec &m, const Grids &grids, V3 a, V3 b, Smp &smp)
 {
     if(m.type == MEDIUM_HOMOGENEOUS)
     {
@@ -256,7 +321,7 @@ BTRC_HD V3 medium_tr(const MediumRec &m, const float *voxels, V3 a, V3 b, Smp &s
     float result = 1.0f;
     V3 uvw;
     float density;
-    while(grid_track_step(m, voxels, g, smp, &uvw, &density))
+    while(grid_track_step(m, grids, g, smp, &uvw, &density))
         result = result * (1.0f - density * m.inv_max_density);
     return v3s(result);
 }

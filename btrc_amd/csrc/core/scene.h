@@ -97,7 +97,7 @@ struct SceneView
     // vacuum) and id n + 1 stands for "no medium"
     int32_t medium_count;
     const MediumRec *media;
-    const float *voxels;
+    Grids grids;
     TextureView tex;
     // the IBL's tile probabilities and their alias table (lut_w * lut_h each)
     const float *env_probs;

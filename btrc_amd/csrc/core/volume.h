@@ -37,14 +37,14 @@ struct VolumeRec
     int32_t ax, ay, az;                 // albedo grid (3 floats per voxel); 0: constant
     uint32_t albedo_offset;
     float albedo[3];
-    float pad;
+    uint32_t brick_offset;              // the density grid's first brick
 };
 
 struct VolumeView
 {
     const VolumeRec *vols;
     int32_t count;
-    const float *voxels;
+    Grids grids;
 };
 
 BTRC_HD float dot3(const float *a, V3 b) { return a[0] * b.x + a[1] * b.y + a[2] * b.z; }
@@ -130,14 +130,14 @@ BTRC_HD float volume_density(const VolumeView &vv, const VolumeRec &v, V3 uvw)
 {
     if(v.nx == 0)
         return v.sigma_t;
-    return grid_lookup(vv.voxels + v.density_offset, v.nx, v.ny, v.nz, 1, 0, uvw);
+    return brick_lookup(vv.grids.bricks + (size_t)v.brick_offset * BRICK_FLOATS, v.nx, v.ny, v.nz, uvw);
 }
 
 BTRC_HD V3 volume_albedo(const VolumeView &vv, const VolumeRec &v, V3 uvw)
 {
     if(v.ax == 0)
         return v3(v.albedo[0], v.albedo[1], v.albedo[2]);
-    const float *g = vv.voxels + v.albedo_offset;
+    const float *g = vv.grids.voxels + v.albedo_offset;
     return v3(grid_lookup(g, v.ax, v.ay, v.az, 3, 0, uvw), grid_lookup(g, v.ax, v.ay, v.az, 3, 1, uvw),
               grid_lookup(g, v.ax, v.ay, v.az, 3, 2, uvw));
 }

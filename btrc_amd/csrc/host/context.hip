@@ -264,6 +264,7 @@ struct btrc_ctx
     DevBuf<AliasUnit> alias;
     DevBuf<MediumRec> media;
     DevBuf<float> voxels;
+    DevBuf<float> bricks;             // density grids, 3 x 3 x 3 voxels a line
     DevBuf<VolumeRec> volumes;
     int32_t volume_count = 0;
     float world_lo[3] = { 0, 0, 0 }, world_hi[3] = { 0, 0, 0 }; // triangles and volume primitives
@@ -424,11 +425,11 @@ struct btrc_ctx
         v.instance_count = instance_count;
         v.medium_count = medium_count;
         v.media = media.ptr;
-        v.voxels = voxels.ptr;
+        v.grids = Grids{ voxels.ptr, bricks.ptr };
         v.tex = TextureView{ textures.ptr, texels8.ptr, texels32.ptr, tex_decode.ptr };
         v.env_probs = env_probs.ptr;
         v.env_alias = env_alias.ptr;
-        v.vol = VolumeView{ volumes.ptr, volume_count, voxels.ptr };
+        v.vol = VolumeView{ volumes.ptr, volume_count, Grids{ voxels.ptr, bricks.ptr } };
         v.world_diagonal = 0.0f; // set per render from the cameras
         return v;
     }
@@ -1111,6 +1112,12 @@ void upload_scene(btrc_ctx *ctx, const btrc_scene_desc *sd)
     std::vector<uint32_t> medium_id(R);
     std::vector<MediumRec> media(R);
     std::vector<float> voxels;
+    uint64_t brick_total = 0; // of all density grids
+    auto add_bricks = [&](int32_t nx, int32_t ny, int32_t nz) {
+        const uint64_t first = brick_total;
+        brick_total += (uint64_t)brick_count(nx) * (uint64_t)brick_count(ny) * (uint64_t)brick_count(nz);
+        return (uint32_t)first;
+    };
     for(int32_t rank = 0; rank < R; ++rank)
     {
         const int32_t i = order[rank];
@@ -1146,6 +1153,7 @@ void upload_scene(btrc_ctx *ctx, const btrc_scene_desc *sd)
             m.nz = nz;
             float mx = -MAX_FLOAT;
             m.density_offset = (uint32_t)voxels.size();
+            m.brick_offset = add_bricks(nx, ny, nz);
             for(size_t v = 0; v < nv; ++v)
             {
                 const float x = md.sigma_t_grid[v];
@@ -1215,6 +1223,7 @@ void upload_scene(btrc_ctx *ctx, const btrc_scene_desc *sd)
                 throw InvalidArg(name + ": voxel grids too large");
             v.nx = nx; v.ny = ny; v.nz = nz;
             v.density_offset = (uint32_t)voxels.size();
+            v.brick_offset = add_bricks(nx, ny, nz);
             float mx = vd.sigma_t_grid[0];
             for(size_t k = 0; k < nv; ++k)
             {
@@ -1388,6 +1397,19 @@ void upload_scene(btrc_ctx *ctx, const btrc_scene_desc *sd)
     ctx->alias.upload(alias_units.data(), alias_units.size(), s);
     ctx->media.upload(media.data(), media.size(), s);
     ctx->voxels.upload(voxels.data(), voxels.size(), s);
+    ctx->bricks.alloc((size_t)brick_total * BRICK_FLOATS);
+    auto make_bricks = [&](const auto &r) {
+        launch_make_bricks(s, ctx->voxels.ptr + r.density_offset, r.nx, r.ny, r.nz,
+                           (uint64_t)brick_count(r.nx) * brick_count(r.ny) * brick_count(r.nz),
+                           ctx->bricks.ptr + (size_t)r.brick_offset * BRICK_FLOATS);
+        BTRC_HIP_CHECK(hipGetLastError());
+    };
+    for(const MediumRec &m : media)
+        if(m.type == BTRC_MEDIUM_HETEROGENEOUS)
+            make_bricks(m);
+    for(const VolumeRec &v : vols)
+        if(v.nx > 0)
+            make_bricks(v);
     ctx->volumes.upload(vols.data(), vols.size(), s);
     ctx->textures.upload(texs.data(), texs.size(), s);
     ctx->texels8.upload(tex8.data(), tex8.size(), s);

@@ -319,6 +319,9 @@ void launch_envir_table(hipStream_t s, const TextureView &tv, int32_t tex, int32
 // the environment light's eval_le, pdf_li and sample_li: 12 floats per query
 void launch_envir_eval(hipStream_t s, const SceneView &sv, const float *dirs, const float *sam, int32_t n, float *out);
 void launch_texture_eval(hipStream_t s, const TextureView &tv, int32_t id, const float2 *uv, int32_t n, float4 *out);
+// a density grid's bricks (brick_count per axis, brick_lookup) from its voxels
+void launch_make_bricks(hipStream_t s, const float *grid, int32_t nx, int32_t ny, int32_t nz, uint64_t bricks,
+                        float *out);
 // the Halton sampler's first-digit tables of `count` dimensions
 void launch_halton_tables(hipStream_t s, const HaltonDim *dims, int32_t count, uint16_t *values);
 void launch_volume_eval(hipStream_t s, const VolumeView &vv, const float4 *seg, const uint2 *seed, int32_t n,

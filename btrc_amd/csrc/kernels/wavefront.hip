@@ -9,6 +9,8 @@
 // bounces. Queue pushes are aggregated per wavefront: one atomic per wave.
 #include "wavefront.h"
 
+#include <algorithm>
+
 namespace btrc {
 
 __constant__ PrimeTable c_primes = make_prime_table();
@@ -960,7 +962,7 @@ __global__ void __launch_bounds__(MEDIUM_BLOCK) k_medium_track(const RenderConst
             const MediumRec &m = sv.media[med];
             V3 uvw;
             float density;
-            const bool inside = grid_track_step(m, sv.voxels, g, hs, &uvw, &density);
+            const bool inside = grid_track_step(m, sv.grids, g, hs, &uvw, &density);
             if(sampling)
             {
                 bool done = !inside;
@@ -969,7 +971,7 @@ __global__ void __launch_bounds__(MEDIUM_BLOCK) k_medium_track(const RenderConst
                     MediumSample ms;
                     ms.scattered = true;
                     ms.position = g.a + g.t * g.world_step;
-                    ms.color = grid_albedo(m, sv.voxels, uvw);
+                    ms.color = grid_albedo(m, sv.grids, uvw);
                     ms.g = m.g;
                     record_scatter(scatter, i, ms);
                     scattered = true;
@@ -1051,8 +1053,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))
                 else
                 {
                     const MediumRec &m = sv.media[med];
-                    ms = medium_sample(m, sv.voxels, o, end, hs);
-                    trv = medium_tr(m, sv.voxels, o, end, hs);
+                    ms = medium_sample(m, sv.grids, o, end, hs);
+                    trv = medium_tr(m, sv.grids, o, end, hs);
                 }
                 const float4 le4 = path.bsdf_le[ps];
                 path.bsdf_le[ps] = f4(xyz(le4) * trv, le4.w);
@@ -1192,7 +1194,7 @@ struct ShadowSink
                 else if(med < (uint32_t)sv.medium_count)
                 {
                     TrSampler ts = TrSampler::start(shadow.seed[i]);
-                    beta = beta * medium_tr(sv.media[med], sv.voxels, o, o + xyz(dd) * dd.w, ts);
+                    beta = beta * medium_tr(sv.media[med], sv.grids, o, o + xyz(dd) * dd.w, ts);
                 }
                 else if(med == (uint32_t)sv.medium_count && sv.vol.count > 0)
                 {
@@ -1381,6 +1383,16 @@ __global__ void k_texture_eval(TextureView tv, int32_t id, const float2 *uv, int
         out[i] = tex_sample(tv, id, uv[i].x, uv[i].y);
 }
 
+// a density grid's bricks, a thread per float
+__global__ void k_make_bricks(const float *grid, int32_t nx, int32_t ny, int32_t nz, uint64_t n, float *bricks)
+{
+    for(uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x)
+    {
+        const uint32_t e = (uint32_t)(i % BRICK_FLOATS);
+        bricks[i] = e < 27 ? brick_element(grid, nx, ny, nz, (uint32_t)(i / BRICK_FLOATS), e) : 0.0f;
+    }
+}
+
 __global__ void k_medium_eval(SceneView sv, int32_t med, const float4 *seg, const uint2 *seed, int32_t n, float *out)
 {
     const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1390,8 +1402,8 @@ __global__ void k_medium_eval(SceneView sv, int32_t med, const float4 *seg, cons
     const V3 a = xyz(a4), b = xyz(a4) + xyz(d4) * d4.w;
     TrSampler smp = TrSampler::start(seed[i]);
     const MediumRec &m = sv.media[med];
-    const MediumSample ms = medium_sample(m, sv.voxels, a, b, smp);
-    const V3 tr = medium_tr(m, sv.voxels, a, b, smp);
+    const MediumSample ms = medium_sample(m, sv.grids, a, b, smp);
+    const V3 tr = medium_tr(m, sv.grids, a, b, smp);
     float *o = out + 10 * (size_t)i;
     o[0] = ms.scattered ? 1.0f : 0.0f;
     o[1] = ms.position.x; o[2] = ms.position.y; o[3] = ms.position.z;
@@ -1669,6 +1681,14 @@ void launch_sample_rows(hipStream_t s, const HaltonConsts &hc, const HaltonTable
 {
     hipLaunchKernelGGL(k_sample_rows, dim3(samples * (ROW_CELLS / 64), (dims + ROW_TILE - 1) / ROW_TILE), dim3(256), 0,
                        s, hc, tab, sample, dims, rows);
+}
+
+void launch_make_bricks(hipStream_t s, const float *grid, int32_t nx, int32_t ny, int32_t nz, uint64_t bricks,
+                        float *out)
+{
+    const uint64_t n = bricks * BRICK_FLOATS;
+    const int blocks = (int)std::min<uint64_t>((n + 255) / 256, 1u << 16);
+    hipLaunchKernelGGL(k_make_bricks, dim3(blocks), dim3(256), 0, s, grid, nx, ny, nz, n, out);
 }
 
 void launch_halton_tables(hipStream_t s, const HaltonDim *dims, int32_t count, uint16_t *values)
