@@ -1844,7 +1844,8 @@ SampleRows plan_sample_rows(btrc_ctx *ctx, const btrc_render_params *p, const st
         return r;
     r.samples = (int32_t)std::min<int64_t>(p->spp, fit);
     r.dims = (int32_t)dims;
-    const size_t floats = (size_t)r.samples * ROW_CELLS * dims;
+    // the tracking kernel loads a chunk of a row past its end
+    const size_t floats = (size_t)r.samples * ROW_CELLS * dims + 16;
     if(ctx->sample_rows.count < floats)
     {
         try
