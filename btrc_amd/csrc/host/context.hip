@@ -2072,6 +2072,7 @@ void render(btrc_ctx *ctx, const btrc_render_params *p, int32_t view_count, cons
         rc.total = window_total;
         *ctx->rc_host = rc;
         BTRC_HIP_CHECK(hipMemcpyAsync(ctx->rc_dev.ptr, ctx->rc_host, sizeof(RenderConsts), hipMemcpyHostToDevice, s));
+        launch_turn(s, rcd, ctx->wc(), p->state_count, 0, true);
         if(rows.samples > 0)
         {
             launch_sample_rows(s, views[0].halton, rc.halton, rc.row_sample, samples, rows.dims, ctx->sample_rows.ptr);
@@ -2088,31 +2089,47 @@ void render(btrc_ctx *ctx, const btrc_render_params *p, int32_t view_count, cons
     int64_t captured = 0;
     const auto t0 = std::chrono::steady_clock::now();
     int cur = 0;
-    // even: a block of bounces ends on the pool side it began with
-    const int check_every = ctx->tuning.graph_bounces > 0 ? ctx->tuning.graph_bounces : 4;
+    // Bounces per captured block, even: a block ends on the pool side it began
+    // with. A frame whose paths all fit the pool needs no more than `bounces`
+    // (every bounce deepens every path that goes on, and none goes on at the
+    // larger of the two depths): up to ONE_BLOCK_BOUNCES of them run as one
+    // block with one read-back, generating in the first bounce only.
+    constexpr int ONE_BLOCK_BOUNCES = 10;
+    int64_t bounces = (int64_t)std::max(p->min_depth, p->max_depth) + 1;
+    if(nrc_on && (!ctx->nrc.params.train || ctx->nrc.params.train_depth > 0))
+    {
+        // the cache ends rendered paths at its query depth and training paths
+        // at theirs
+        const int32_t tail = ctx->nrc.params.train ? ctx->nrc.params.train_depth : 0;
+        bounces = std::min<int64_t>(bounces, (int64_t)std::max(ctx->nrc.params.query_depth, tail) + 1);
+    }
+    const bool one_block = ctx->tuning.graph_bounces == 0 && total <= (uint64_t)p->state_count &&
+                           bounces <= ONE_BLOCK_BOUNCES && (rows.samples == 0 || rows.samples == p->spp);
+    const int check_every = one_block ? (int)bounces : ctx->tuning.graph_bounces > 0 ? ctx->tuning.graph_bounces : 4;
 
-    // one bounce: plan, generate, trace, [medium], shade, shadow. With
-    // `overlap` the shadow rays go to the shadow stream and are traced beside
-    // the next bounce's plan, generate and trace; the next bounce's medium
-    // and shade stages (which write the film, the radiance sums and the
-    // shadow queue again) wait for them.
+    // one bounce: generate, trace, [medium], shade, shadow, then the turn to
+    // the next. With `overlap` the shadow rays go to the shadow stream and are
+    // traced beside the next bounce's generate and trace; the next bounce's
+    // medium and shade stages (which write the film, the radiance sums and
+    // the shadow queue again) wait for them.
     bool shadow_open = false; // a shadow launch on the shadow stream not yet joined
     auto join_shadow = [&] {
         if(shadow_open)
             BTRC_HIP_CHECK(hipStreamWaitEvent(s, ctx->shadow_done, 0));
         shadow_open = false;
     };
-    auto enqueue_bounce = [&](int side, bool timed, bool overlap) {
+    auto enqueue_bounce = [&](int k, bool timed, bool overlap) {
+        const int side = k & 1;
         PathSOA path = ctx->pool[side].view();
         PathSOA next = ctx->pool[side ^ 1].view();
-        launch_plan(s, rcd, ctx->wc(), p->state_count, side);
         auto run = [&](int stage, auto &&fn) {
             if(timed)
                 timer.run(stage, fn);
             else
                 fn();
         };
-        run(STAGE_GENERATE, [&] { launch_generate(s, grid256, sampler, rcd, ctx->wc(), path); });
+        if(k == 0 || !one_block)
+            run(STAGE_GENERATE, [&] { launch_generate(s, grid256, sampler, rcd, ctx->wc(), path); });
         run(STAGE_TRACE, [&] { launch_trace_extension(s, ctx->trace_grid, ctx->trace_sched(false), ts, ctx->wc(), path, hit, ovf); });
         join_shadow();
         if(media)
@@ -2132,7 +2149,35 @@ void render(btrc_ctx *ctx, const btrc_render_params *p, int32_t view_count, cons
         }
         else
             run(STAGE_SHADOW, [&] { launch_shadow(s, shadow_grid, ctx->trace_sched(true), media, ts, sv, ctx->wc(), sh, fv, shadow_ovf, side); });
-        launch_end_iteration(s, ctx->wc(), side);
+        launch_turn(s, rcd, ctx->wc(), p->state_count, side ^ 1, false);
+    };
+    // a block of bounces whose launches do not fill the GPU: a bounce's shadow
+    // rays share a launch with the next bounce's extension rays
+    const int64_t most_rays = (int64_t)std::min<uint64_t>((uint64_t)p->state_count, total);
+    auto small_grid = [&](int full) {
+        return (int)std::min<int64_t>(std::min(full, ctx->cu_count * TRACE_WAVES_ANY), (most_rays + 63) / 64);
+    };
+    auto enqueue_small_block = [&] {
+        for(int k = 0; k < check_every; ++k)
+        {
+            const int side = k & 1;
+            PathSOA path = ctx->pool[side].view();
+            PathSOA next = ctx->pool[side ^ 1].view();
+            if(k == 0 || !one_block)
+                launch_generate(s, grid256, sampler, rcd, ctx->wc(), path);
+            if(k == 0)
+                launch_trace_extension(s, small_grid(ctx->trace_grid), ctx->trace_sched(false), ts, ctx->wc(), path, hit, ovf);
+            else
+                launch_trace_both(s, small_grid(ctx->trace_grid), small_grid(shadow_grid), ctx->two_level, media, ts, sv,
+                                  ctx->wc(), path, hit, sh, fv, ovf, shadow_ovf, side);
+            if(media)
+                launch_medium(s, grid256, ctx->cu_count * MEDIUM_TRACK_WAVES_PER_CU, sampler, rcd, sv, ctx->wc(), path,
+                              hit, ctx->medium_scatter.ptr, next, sh, fv, side);
+            launch_shade(s, grid256, sampler, rcd, sv, ctx->wc(), path, hit, next, sh, fv, nv, side);
+            launch_turn(s, rcd, ctx->wc(), p->state_count, side ^ 1, false);
+        }
+        launch_shadow(s, small_grid(shadow_grid), ctx->trace_sched(true), media, ts, sv, ctx->wc(), sh, fv, shadow_ovf,
+                      (check_every - 1) & 1);
     };
 
     if(ctx->tuning.launch_graph && !timer.enabled && !capture)
@@ -2150,9 +2195,12 @@ void render(btrc_ctx *ctx, const btrc_render_params *p, int32_t view_count, cons
         // the shadow stream pays off once a bounce fills the GPU: the event
         // hand-offs cost ~6 us per bounce (256^2 frames: +8 %), the overlap
         // saves ~7 % of a 1080p frame
-        const bool overlap = std::min<uint64_t>((uint64_t)p->state_count, total) >= (1u << 20);
-        const int32_t ints[9] = { grid256, ctx->trace_grid, ctx->trace_sched(false), ctx->trace_sched(true),
-                                  sampler, p->state_count, media ? 1 : 0, check_every, overlap ? 1 : 0 };
+        const bool overlap = most_rays >= (1 << 20);
+        // (the joint launch is compiled for the default schedules)
+        const bool small = !overlap && !(ctx->trace_sched(false) & SCHED_POSTPONE) && !(ctx->trace_sched(true) & SCHED_POSTPONE);
+        const int32_t ints[12] = { grid256, ctx->trace_grid, ctx->trace_sched(false), ctx->trace_sched(true),
+                                   sampler, p->state_count, media ? 1 : 0, check_every, overlap ? 1 : 0, small ? 1 : 0,
+                                   small ? small_grid(ctx->trace_grid) : 0, one_block ? 1 : 0 };
         add(ints);
         int g = -1;
         for(int k = 0; k < 2; ++k)
@@ -2168,9 +2216,14 @@ void render(btrc_ctx *ctx, const btrc_render_params *p, int32_t view_count, cons
             ctx->loop_key[g].clear();
             hipGraph_t graph = nullptr;
             BTRC_HIP_CHECK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-            for(int k = 0; k < check_every; ++k)
-                enqueue_bounce(k & 1, false, overlap);
-            join_shadow();
+            if(small)
+                enqueue_small_block();
+            else
+            {
+                for(int k = 0; k < check_every; ++k)
+                    enqueue_bounce(k, false, overlap);
+                join_shadow();
+            }
             BTRC_HIP_CHECK(hipStreamEndCapture(s, &graph));
             const hipError_t e = hipGraphInstantiate(&ctx->loop_exec[g], graph, nullptr, nullptr, 0);
             (void)hipGraphDestroy(graph);
@@ -2193,6 +2246,8 @@ void render(btrc_ctx *ctx, const btrc_render_params *p, int32_t view_count, cons
             reporter_stage.progress(hc, total);
             if(hc.generated == window_total && hc.active == 0)
                 break;
+            if(one_block)
+                throw std::logic_error("a path went on past the deepest bounce");
         }
     }
     else
@@ -2203,7 +2258,6 @@ void render(btrc_ctx *ctx, const btrc_render_params *p, int32_t view_count, cons
             throw Stopped("render stopped");
         PathSOA path = ctx->pool[cur].view();
         PathSOA next = ctx->pool[cur ^ 1].view();
-        launch_plan(s, rcd, ctx->wc(), p->state_count, cur);
         timer.run(STAGE_GENERATE, [&] { launch_generate(s, grid256, sampler, rcd, ctx->wc(), path); });
         timer.run(STAGE_TRACE, [&] { launch_trace_extension(s, ctx->trace_grid, ctx->trace_sched(false), ts, ctx->wc(), path, hit, ovf); });
         if(capture && (int64_t)iter < capture_bounces && captured < capture_max)
@@ -2244,7 +2298,7 @@ void render(btrc_ctx *ctx, const btrc_render_params *p, int32_t view_count, cons
             });
         timer.run(STAGE_SHADE, [&] { launch_shade(s, grid256, sampler, rcd, sv, ctx->wc(), path, hit, next, sh, fv, nv, cur); });
         timer.run(STAGE_SHADOW, [&] { launch_shadow(s, shadow_grid, ctx->trace_sched(true), media, ts, sv, ctx->wc(), sh, fv, shadow_ovf, cur); });
-        launch_end_iteration(s, ctx->wc(), cur);
+        launch_turn(s, rcd, ctx->wc(), p->state_count, cur ^ 1, false);
         BTRC_HIP_CHECK(hipGetLastError());
         cur ^= 1;
         if((iter + 1) % check_every == 0)

@@ -37,6 +37,10 @@ constexpr int TRACE_BLOCK = 64;   // one wavefront per workgroup
 // stop at 20.
 constexpr int SHORT_STACK_CLOSEST = 12, SHORT_STACK_ANY = 16, SHORT_STACK_TWO = 16;
 constexpr int SHORT_STACK_MIN = 12; // what the overflow area is sized by
+constexpr int short_stack(bool any, bool two)
+{
+    return two ? SHORT_STACK_TWO : any ? SHORT_STACK_ANY : SHORT_STACK_CLOSEST;
+}
 // Idle lanes that trigger a refill: 24 for one level (35.8 / 34.7 / 33.8 ms of
 // closest-hit traversal per 1080p, 32 spp field frame at 12 / 16 / 24), 16 for
 // two (12.35 against 12.5 ms at 24 per four-view frame)
@@ -157,8 +161,8 @@ struct HitRecord
 // geometry's tree; popping CODE_EXIT restores the world ray.
 //
 // Traces rays [0, n): each wavefront's first TRACE_BLOCK rays by its
-// workgroup index, the rest [gridDim.x * TRACE_BLOCK, n) in granules of
-// GRANULE rays dealt round robin to C = min(COUNTER_STRIPES, gridDim.x)
+// workgroup index, the rest [grid * TRACE_BLOCK, n) in granules of
+// GRANULE rays dealt round robin to C = min(COUNTER_STRIPES, grid)
 // chunks, chunk k's granules handed out by counter fetch[k * COUNTER_STRIDE]
 // (all FETCH_WORDS words start at 0) to the wavefronts of workgroups
 // b = k (mod C). Sink provides
@@ -178,15 +182,19 @@ struct HitRecord
 // distances by one fused multiply-add a plane, triangle rows in the ray's axis
 // order, pushes and pops without overflow handling while no lane is deep, and
 // every load of a step issued together.
+//
+// block, grid: this workgroup's index among the workgroups that trace these
+// rays, and their number (a launch may hold two sets). s_stack: LDS of
+// short_stack(ANY, TWO) * TRACE_BLOCK entries.
 template<int TRI, bool ANY, bool POSTPONE, bool TWO, class Sink>
 __device__ __forceinline__ void trace_persistent(
-    const TraceScene &sc, Sink &sink, int32_t n, uint32_t *fetch, const TraceOverflow &ovf)
+    const TraceScene &sc, Sink &sink, int32_t n, uint32_t *fetch, const TraceOverflow &ovf, uint32_t block, uint32_t grid,
+    uint2 *s_stack)
 {
     constexpr int REFILL_MIN = TWO ? REFILL_MIN_TWO : REFILL_MIN_ONE;
-    constexpr int SHORT_STACK = TWO ? SHORT_STACK_TWO : ANY ? SHORT_STACK_ANY : SHORT_STACK_CLOSEST;
-    __shared__ uint2 s_stack[SHORT_STACK * TRACE_BLOCK];
+    constexpr int SHORT_STACK = short_stack(ANY, TWO);
     const int lane = (int)threadIdx.x;
-    const int gl = (int)(blockIdx.x * TRACE_BLOCK + threadIdx.x);
+    const int gl = (int)(block * TRACE_BLOCK + threadIdx.x);
     const uint64_t lanes_below = (1ull << lane) - 1ull;
 
     bool active = false;
@@ -214,13 +222,13 @@ __device__ __forceinline__ void trace_persistent(
     // contiguous chunks per XCD, the dry ones helped out, left the field
     // frame's traversal as it was and slowed smaller frames by up to a
     // fifth). A wavefront keeps the rest of its granule for its next refill.
-    const uint32_t static_span = gridDim.x * (uint32_t)TRACE_BLOCK;
-    const uint32_t chunks = min((uint32_t)COUNTER_STRIPES, gridDim.x); // every chunk has wavefronts
-    const uint32_t home = blockIdx.x % chunks;
+    const uint32_t static_span = grid * (uint32_t)TRACE_BLOCK;
+    const uint32_t chunks = min((uint32_t)COUNTER_STRIPES, grid); // every chunk has wavefronts
+    const uint32_t home = block % chunks;
     uint32_t *counter = fetch + home * COUNTER_STRIDE;
     // wavefront-uniform: reserved rays not yet handed out, whether the home
     // chunk has run dry, and whether no ray is left for this wavefront
-    uint32_t res_lo = min((uint32_t)n, blockIdx.x * (uint32_t)TRACE_BLOCK);
+    uint32_t res_lo = min((uint32_t)n, block * (uint32_t)TRACE_BLOCK);
     uint32_t res_hi = min((uint32_t)n, res_lo + (uint32_t)TRACE_BLOCK);
     bool dry = static_span >= (uint32_t)n;
     bool exhausted = dry && res_lo == res_hi;

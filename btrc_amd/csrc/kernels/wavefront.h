@@ -276,7 +276,8 @@ enum : int
 };
 
 // parity: the bounce's parity (the pool side it reads)
-void launch_plan(hipStream_t s, const RenderConsts *rc, WaveCounters *c, int32_t state_count, int parity);
+// before the bounce of this parity (first: no bounce came before it)
+void launch_turn(hipStream_t s, const RenderConsts *rc, WaveCounters *c, int32_t state_count, int parity, bool first);
 // fills `samples` * ROW_CELLS sample rows from first sample `sample` on
 void launch_sample_rows(hipStream_t s, const HaltonConsts &hc, const HaltonTables &tab, int32_t sample, int32_t samples,
                         int32_t dims, float *rows);
@@ -296,7 +297,10 @@ void launch_medium(hipStream_t s, int grid, int track_grid, int sampler, const R
                    ShadowSOA shadow, FilmView film, int parity);
 void launch_shadow(hipStream_t s, int grid, int sched, bool media, const TraceScene &ts, const SceneView &sv,
                    WaveCounters *c, ShadowSOA shadow, FilmView film, const TraceOverflow &ovf, int parity);
-void launch_end_iteration(hipStream_t s, WaveCounters *c, int parity);
+// the extension rays of the bounce of this parity and the shadow rays of the one before it
+void launch_trace_both(hipStream_t s, int ext_grid, int shadow_grid, bool two_level, bool media, const TraceScene &ts,
+                       const SceneView &sv, WaveCounters *c, PathSOA path, HitSOA hit, ShadowSOA shadow,
+                       FilmView film, const TraceOverflow &ovf, const TraceOverflow &shadow_ovf, int parity);
 void launch_resolve(hipStream_t s, int mode, const float *value, int32_t pixels, float inv_weight, float4 *out);
 
 // ray batches of the traversal entry points: o.xyz/tmin and d.xyz/tmax

@@ -252,43 +252,90 @@ struct TrSampler
     __device__ float get1d() { return pcg32_uniform_float(rng); }
 };
 
-// ---------------------------------------------------------------- plan
+// ---------------------------------------------------------------- turn
 
-// GeneratePipeline::generate's refill rule (generate.cpp:140-176), evaluated
-// on the device: refill when at least half of the pool is free or when all
-// remaining paths fit.
-__global__ void k_plan(const RenderConsts *rc, WaveCounters *c, int32_t state_count, int parity)
+// Between two bounces, one wavefront: the states that the bounce of the other
+// parity pushed become the current pool side (one segment per stripe), its
+// rays are counted, and the bounce of `parity` is planned. `first`: there was
+// no bounce before.
+//
+// The plan is GeneratePipeline::generate's refill rule (generate.cpp:140-176):
+// refill when at least half of the pool is free or when all remaining paths
+// fit. The generated states form the last segment.
+//
+// Latency-bound: the sixteen stripes' counters are read and written by
+// sixteen lanes at once (two launches of one lane each took 3.6 + 4.0 us a
+// bounce, this one 3).
+__global__ void __launch_bounds__(64) k_turn(const RenderConsts *rc, WaveCounters *c, int32_t state_count, int parity,
+                                             int first)
 {
-    const uint64_t total = rc->total;
     QueueState *q = queue_state(c);
-    const int32_t active = c->active;
-    const int64_t rest = (int64_t)state_count - active;
-    int64_t fresh = 0;
-    if(c->generated < total && rest > 0)
+    const int lane = (int)threadIdx.x;
+    const uint64_t total = rc->total;
+    const uint64_t generated = c->generated;
+    const int32_t old_stripe = q->stripe[parity ^ 1];
+    int32_t states = 0, shadows = 0;
+    if(lane < COUNTER_STRIPES)
     {
-        const int64_t unfinished = (int64_t)(total - c->generated);
-        if(!(unfinished > rest && rest + rest < state_count))
-            fresh = unfinished < rest ? unfinished : rest;
-    }
-    for(int k = 0; k < FETCH_WORDS; k += COUNTER_STRIDE)
-    {
+        const int k = lane * COUNTER_STRIDE;
+        if(!first)
+        {
+            states = q->next_n[k];
+            shadows = q->shadow_n[parity ^ 1][k];
+        }
+        else
+        {
+            q->shadow_n[parity ^ 1][k] = 0;
+            q->shadow_fetch[parity ^ 1][k] = 0;
+        }
+        // the next-state and fetch counters restart, and the shadow counters
+        // of this parity (the rays pushed two bounces ago have been traced)
+        q->next_n[k] = 0;
+        q->shadow_n[parity][k] = 0;
+        q->shadow_fetch[parity][k] = 0;
         q->trace_fetch[k] = 0;
         q->medium_fetch[k] = 0;
     }
-    // the generated states form the last segment of the current side
-    const int32_t n = active + (int32_t)fresh;
-    q->pool_first[COUNTER_STRIPES] = pool_gen_slot(state_count);
-    q->pool_prefix[COUNTER_STRIPES] = active;
-    q->pool_prefix[COUNTER_STRIPES + 1] = n;
-    // this bounce's pushes: COUNTER_STRIPES stripes over its n inputs
-    const int32_t per = (n + COUNTER_STRIPES - 1) / COUNTER_STRIPES;
-    q->stripe[parity] = per > 0 ? (per + 63) / 64 * 64 : 64;
-    c->gen_offset = active;
-    c->gen_count = (int32_t)fresh;
-    c->gen_base = c->generated;
-    c->generated += (uint64_t)fresh;
-    c->active = n;
-    c->ext_rays += (uint64_t)n;
+    int32_t upto = states; // states of stripes 0 .. lane
+    for(int step = 1; step < COUNTER_STRIPES; step *= 2)
+    {
+        const int32_t below = __shfl_up(upto, step);
+        if(lane >= step)
+            upto += below;
+        shadows += __shfl_xor(shadows, step);
+    }
+    const int32_t active = __shfl(upto, COUNTER_STRIPES - 1);
+    if(lane < COUNTER_STRIPES)
+    {
+        q->pool_first[lane] = lane * old_stripe;
+        q->pool_prefix[lane] = upto - states;
+    }
+    if(lane == 0)
+    {
+        const int64_t rest = (int64_t)state_count - active;
+        int64_t fresh = 0;
+        if(generated < total && rest > 0)
+        {
+            const int64_t unfinished = (int64_t)(total - generated);
+            if(!(unfinished > rest && rest + rest < state_count))
+                fresh = unfinished < rest ? unfinished : rest;
+        }
+        const int32_t n = active + (int32_t)fresh;
+        q->pool_first[COUNTER_STRIPES] = pool_gen_slot(state_count);
+        q->pool_prefix[COUNTER_STRIPES] = active;
+        q->pool_prefix[COUNTER_STRIPES + 1] = n;
+        // this bounce's pushes: COUNTER_STRIPES stripes over its n inputs
+        const int32_t per = (n + COUNTER_STRIPES - 1) / COUNTER_STRIPES;
+        q->stripe[parity] = per > 0 ? (per + 63) / 64 * 64 : 64;
+        c->gen_offset = active;
+        c->gen_count = (int32_t)fresh;
+        c->gen_base = generated;
+        c->generated = generated + (uint64_t)fresh;
+        c->active = n;
+        c->ext_rays += (uint64_t)n;
+        c->shadow_rays += (uint64_t)shadows;
+        c->iterations += first ? 0 : 1;
+    }
 }
 
 // ---------------------------------------------------------------- sample rows
@@ -459,10 +506,11 @@ template<int SCHED>
 __global__ void __launch_bounds__(TRACE_BLOCK) TRACE_WAVES(SCHED, false, false) k_trace_extension(
     TraceScene ts, WaveCounters *c, PathSOA path, HitSOA hit, TraceOverflow ovf)
 {
+    __shared__ uint2 s_stack[short_stack(false, (SCHED & SCHED_TWO_LEVEL) != 0) * TRACE_BLOCK];
     QueueState *q = queue_state(c);
     ExtensionSink sink{ path, hit, q };
     trace_persistent<TRI_WATERTIGHT, false, (SCHED & SCHED_POSTPONE) != 0, (SCHED & SCHED_TWO_LEVEL) != 0>(
-        ts, sink, c->active, q->trace_fetch, ovf);
+        ts, sink, c->active, q->trace_fetch, ovf, blockIdx.x, gridDim.x, s_stack);
 }
 
 // ---------------------------------------------------------------- shade
@@ -1275,39 +1323,43 @@ template<int SCHED, bool MEDIA>
 __global__ void __launch_bounds__(TRACE_BLOCK) TRACE_WAVES(SCHED, MEDIA, true) k_shadow(
     TraceScene ts, SceneView sv, WaveCounters *c, ShadowSOA shadow, FilmView film, TraceOverflow ovf, int parity)
 {
+    __shared__ uint2 s_stack[short_stack(true, (SCHED & SCHED_TWO_LEVEL) != 0) * TRACE_BLOCK];
     QueueState *q = queue_state(c);
     ShadowSink<MEDIA> sink{ shadow, film, sv, q, parity };
     trace_persistent<TRI_WATERTIGHT, true, (SCHED & SCHED_POSTPONE) != 0, (SCHED & SCHED_TWO_LEVEL) != 0>(
-        ts, sink, shadow_count(q, parity), q->shadow_fetch[parity], ovf);
+        ts, sink, shadow_count(q, parity), q->shadow_fetch[parity], ovf, blockIdx.x, gridDim.x, s_stack);
 }
 
-// ---------------------------------------------------------------- bookkeeping
-
-// the states pushed this bounce become the next bounce's pool side: one
-// segment per stripe, then the (empty) generated segment; the next-state
-// counters restart, and so do the shadow counters of the other parity (the
-// previous bounce's shadow rays were traced before this bounce shaded)
-__global__ void k_end_iteration(WaveCounters *c, int parity)
+// The shadow rays of a bounce (of parity `parity ^ 1`) and the extension rays
+// of the next in one launch: workgroups 0 .. ext_grid - 1 trace the extension
+// rays, the rest the shadow rays. For frames whose launches do not fill the
+// GPU: each leaves most of the time to its longest rays, and here the two run
+// together without the events that two streams would need (6 us a bounce).
+template<bool TWO, bool MEDIA>
+__global__ void __launch_bounds__(TRACE_BLOCK) k_trace_both(
+    TraceScene ts, SceneView sv, WaveCounters *c, PathSOA path, HitSOA hit, ShadowSOA shadow, FilmView film,
+    TraceOverflow ovf, TraceOverflow shadow_ovf, int parity, uint32_t ext_grid)
 {
+    __shared__ uint2 s_stack[short_stack(true, TWO) * TRACE_BLOCK]; // either set's (the closest-hit one is no larger)
+    static_assert(short_stack(false, TWO) <= short_stack(true, TWO), "one LDS stack serves both");
     QueueState *q = queue_state(c);
-    const int32_t stripe = q->stripe[parity];
-    int32_t states = 0, shadows = 0;
-    for(int k = 0; k < COUNTER_STRIPES; ++k)
+    if(blockIdx.x < ext_grid)
     {
-        q->pool_first[k] = k * stripe;
-        q->pool_prefix[k] = states;
-        states += q->next_n[k * COUNTER_STRIDE];
-        shadows += q->shadow_n[parity][k * COUNTER_STRIDE];
-        q->next_n[k * COUNTER_STRIDE] = 0;
-        q->shadow_n[parity ^ 1][k * COUNTER_STRIDE] = 0;
-        q->shadow_fetch[parity ^ 1][k * COUNTER_STRIDE] = 0;
+        ExtensionSink sink{ path, hit, q };
+        trace_persistent<TRI_WATERTIGHT, false, false, TWO>(ts, sink, c->active, q->trace_fetch, ovf, blockIdx.x,
+                                                            ext_grid, s_stack);
     }
-    q->pool_prefix[COUNTER_STRIPES] = states;
-    q->pool_prefix[COUNTER_STRIPES + 1] = states;
-    c->shadow_rays += (uint64_t)shadows;
-    c->active = states;
-    c->iterations += 1;
+    else
+    {
+        const int before = parity ^ 1;
+        ShadowSink<MEDIA> sink{ shadow, film, sv, q, before };
+        trace_persistent<TRI_WATERTIGHT, true, false, TWO>(ts, sink, shadow_count(q, before), q->shadow_fetch[before],
+                                                           shadow_ovf, blockIdx.x - ext_grid, gridDim.x - ext_grid,
+                                                           s_stack);
+    }
 }
+
+// ---------------------------------------------------------------- resolve
 
 // preview resolve, wavefront/preview.cpp:28-80: value / weight (weight =
 // samples per pixel); normals are normalised, or zero when shorter than 1e-3
@@ -1362,7 +1414,9 @@ __global__ void __launch_bounds__(TRACE_BLOCK) TRACE_WAVES(SCHED, false, ANY) k_
     TraceScene ts, const float4 *rays, int32_t n, uint32_t *out, uint32_t *fetch, TraceOverflow ovf)
 {
     BatchSink<ANY> sink{ rays, out };
-    trace_persistent<TRI, ANY, (SCHED & SCHED_POSTPONE) != 0, (SCHED & SCHED_TWO_LEVEL) != 0>(ts, sink, n, fetch, ovf);
+    __shared__ uint2 s_stack[short_stack(ANY, (SCHED & SCHED_TWO_LEVEL) != 0) * TRACE_BLOCK];
+    trace_persistent<TRI, ANY, (SCHED & SCHED_POSTPONE) != 0, (SCHED & SCHED_TWO_LEVEL) != 0>(
+        ts, sink, n, fetch, ovf, blockIdx.x, gridDim.x, s_stack);
 }
 
 // ---------------------------------------------------------------- test hooks
@@ -1584,9 +1638,9 @@ __global__ void k_detmath_eval(int32_t fn, const float *x, const float *y, int32
 
 // ---------------------------------------------------------------- launchers
 
-void launch_plan(hipStream_t s, const RenderConsts *rc, WaveCounters *c, int32_t state_count, int parity)
+void launch_turn(hipStream_t s, const RenderConsts *rc, WaveCounters *c, int32_t state_count, int parity, bool first)
 {
-    hipLaunchKernelGGL(k_plan, dim3(1), dim3(1), 0, s, rc, c, state_count, parity);
+    hipLaunchKernelGGL(k_turn, dim3(1), dim3(64), 0, s, rc, c, state_count, parity, first ? 1 : 0);
 }
 
 void launch_generate(hipStream_t s, int grid, int sampler, const RenderConsts *rc, const WaveCounters *c,
@@ -1678,9 +1732,24 @@ void launch_shadow(hipStream_t s, int grid, int sched, bool media, const TraceSc
         launch_shadow_t<SCHED_EAGER>(s, grid, media, ts, sv, c, shadow, film, ovf, parity);
 }
 
-void launch_end_iteration(hipStream_t s, WaveCounters *c, int parity)
+void launch_trace_both(hipStream_t s, int ext_grid, int shadow_grid, bool two_level, bool media, const TraceScene &ts,
+                       const SceneView &sv, WaveCounters *c, PathSOA path, HitSOA hit, ShadowSOA shadow,
+                       FilmView film, const TraceOverflow &ovf, const TraceOverflow &shadow_ovf, int parity)
 {
-    hipLaunchKernelGGL(k_end_iteration, dim3(1), dim3(1), 0, s, c, parity);
+    const dim3 g(ext_grid + shadow_grid), b(TRACE_BLOCK);
+    const uint32_t e = (uint32_t)ext_grid;
+    if(two_level && media)
+        hipLaunchKernelGGL((k_trace_both<true, true>), g, b, 0, s, ts, sv, c, path, hit, shadow, film, ovf, shadow_ovf,
+                           parity, e);
+    else if(two_level)
+        hipLaunchKernelGGL((k_trace_both<true, false>), g, b, 0, s, ts, sv, c, path, hit, shadow, film, ovf, shadow_ovf,
+                           parity, e);
+    else if(media)
+        hipLaunchKernelGGL((k_trace_both<false, true>), g, b, 0, s, ts, sv, c, path, hit, shadow, film, ovf, shadow_ovf,
+                           parity, e);
+    else
+        hipLaunchKernelGGL((k_trace_both<false, false>), g, b, 0, s, ts, sv, c, path, hit, shadow, film, ovf,
+                           shadow_ovf, parity, e);
 }
 
 void launch_resolve(hipStream_t s, int mode, const float *value, int32_t pixels, float inv_weight, float4 *out)
