@@ -1814,38 +1814,48 @@ std::vector<ViewRec> make_views(btrc_ctx *ctx, const btrc_render_params *p, int3
 
 // Whether a frame reads its Halton numbers from sample rows, and how many
 // samples and dimensions its rows hold (samples 0: the stages run the digit
-// loop). Rows pay off once enough pixels share each: ROWS_MIN_SHARE. They
-// hold every dimension a path can draw: four for the camera, eight per vertex,
-// the last one at the larger of the two depths (all 998 with media, whose tracking steps draw without a bound). Frames of
-// more samples than ROWS_MAX_BYTES holds go through in windows of samples,
-// which needs sample-major paths: one view in uniform order.
-constexpr uint64_t ROWS_MIN_SHARE = 12;
+// loop). Rows hold every dimension a path can draw: four for the camera, eight
+// per vertex of at most `bounces` (all 998 with media, whose tracking steps
+// draw without a bound). They pay off once enough pixels share each
+// (ROWS_MIN_SHARE: 640x360, 14 pixels a row, gains 3 %; 256^2 at 16 spp, 4
+// pixels a row, 1,934 us without and 2,082 with them), and for frames so small
+// that the digit loops' latency counts, not their number (ROWS_SMALL_VALUES: a
+// 320x180 preview's 1.2 million values, 566 us without and 514 with them).
+// Frames of more samples than ROWS_MAX_BYTES holds go through in windows of
+// samples, which needs sample-major paths: one view in uniform order.
+constexpr int64_t ROWS_MIN_SHARE = 12;
+constexpr int64_t ROWS_SMALL_VALUES = 2 << 20;
 constexpr size_t ROWS_MAX_BYTES = (size_t)2 << 30;
 
 struct SampleRows
 {
-    int32_t samples = 0, dims = 0;
+    int32_t samples = 0, dims = 0, width = 0, height = 0;
 };
 
 SampleRows plan_sample_rows(btrc_ctx *ctx, const btrc_render_params *p, const std::vector<ViewRec> &views,
-                            uint64_t pixels, bool media)
+                            uint64_t pixels, bool media, int64_t bounces)
 {
     SampleRows r;
-    if(p->sampler != BTRC_SAMPLER_HALTON || pixels < ROWS_MIN_SHARE * (uint64_t)ROW_CELLS)
+    if(p->sampler != BTRC_SAMPLER_HALTON)
         return r;
     for(const ViewRec &v : views)
-        if(v.width < MAX_HALTON_RESOLUTION || v.height < MAX_HALTON_RESOLUTION)
-            return r; // another stride, other indices
+        if(views.size() > 1 && (v.width < MAX_HALTON_RESOLUTION || v.height < MAX_HALTON_RESOLUTION))
+            return r; // views of several strides: several sets of indices
+    r.width = std::min(views[0].width, MAX_HALTON_RESOLUTION);
+    r.height = std::min(views[0].height, MAX_HALTON_RESOLUTION);
+    const int64_t cells = (int64_t)r.width * r.height;
     const int64_t most = PRIME_TABLE_SIZE - 2;
-    const int64_t need = media ? most : std::min<int64_t>(most, 4 + 8 * ((int64_t)std::max(p->min_depth, p->max_depth) + 1));
+    const int64_t need = media ? most : std::min<int64_t>(most, 4 + 8 * bounces);
     const int64_t dims = (need + 3) / 4 * 4;
-    const int64_t fit = (int64_t)(ROWS_MAX_BYTES / ((size_t)ROW_CELLS * dims * sizeof(float)));
-    if(p->spp > fit && (views.size() > 1 || p->tile))
+    const bool shared = (int64_t)pixels >= ROWS_MIN_SHARE * cells;
+    const bool small = cells * p->spp <= ROWS_SMALL_VALUES / dims;
+    const int64_t fit = (int64_t)(ROWS_MAX_BYTES / ((size_t)cells * dims * sizeof(float)));
+    if((!shared && !small) || (p->spp > fit && (views.size() > 1 || p->tile)))
         return r;
     r.samples = (int32_t)std::min<int64_t>(p->spp, fit);
     r.dims = (int32_t)dims;
     // the tracking kernel loads a chunk of a row past its end
-    const size_t floats = (size_t)r.samples * ROW_CELLS * dims + 16;
+    const size_t floats = (size_t)r.samples * cells * dims + 16;
     if(ctx->sample_rows.count < floats)
     {
         try
@@ -2018,10 +2028,22 @@ void render(btrc_ctx *ctx, const btrc_render_params *p, int32_t view_count, cons
     }
     rc.filter = ctx->filter;
     rc.halton = halton_tables(ctx);
-    const SampleRows rows = plan_sample_rows(ctx, p, views, pixels, media);
+    // no path makes more bounces: each deepens it, and none goes on at the
+    // larger of the two depths
+    int64_t bounces = (int64_t)std::max(p->min_depth, p->max_depth) + 1;
+    if(nrc_on && (!ctx->nrc.params.train || ctx->nrc.params.train_depth > 0))
+    {
+        // the cache ends rendered paths at its query depth and training paths
+        // at theirs
+        const int32_t tail = ctx->nrc.params.train ? ctx->nrc.params.train_depth : 0;
+        bounces = std::min<int64_t>(bounces, (int64_t)std::max(ctx->nrc.params.query_depth, tail) + 1);
+    }
+    const SampleRows rows = plan_sample_rows(ctx, p, views, pixels, media, bounces);
     const int sampler = rows.samples > 0 ? (int)SAMPLER_HALTON_ROWS : (int)p->sampler;
     rc.rows = rows.samples > 0 ? ctx->sample_rows.ptr : nullptr;
     rc.row_dims = rows.dims;
+    rc.row_width = rows.width;
+    rc.row_height = rows.height;
 
     const TraceScene ts = ctx->trace_scene();
     SceneView sv = ctx->scene_view();
@@ -2075,7 +2097,8 @@ void render(btrc_ctx *ctx, const btrc_render_params *p, int32_t view_count, cons
         launch_turn(s, rcd, ctx->wc(), p->state_count, 0, true);
         if(rows.samples > 0)
         {
-            launch_sample_rows(s, views[0].halton, rc.halton, rc.row_sample, samples, rows.dims, ctx->sample_rows.ptr);
+            launch_sample_rows(s, views[0].halton, rc.halton, rows.width, rows.height, rc.row_sample, samples, rows.dims,
+                               ctx->sample_rows.ptr);
             BTRC_HIP_CHECK(hipGetLastError());
         }
         return true;
@@ -2090,19 +2113,10 @@ void render(btrc_ctx *ctx, const btrc_render_params *p, int32_t view_count, cons
     const auto t0 = std::chrono::steady_clock::now();
     int cur = 0;
     // Bounces per captured block, even: a block ends on the pool side it began
-    // with. A frame whose paths all fit the pool needs no more than `bounces`
-    // (every bounce deepens every path that goes on, and none goes on at the
-    // larger of the two depths): up to ONE_BLOCK_BOUNCES of them run as one
-    // block with one read-back, generating in the first bounce only.
+    // with. A frame whose paths all fit the pool needs no more than `bounces`:
+    // up to ONE_BLOCK_BOUNCES of them run as one block with one read-back,
+    // generating in the first bounce only.
     constexpr int ONE_BLOCK_BOUNCES = 10;
-    int64_t bounces = (int64_t)std::max(p->min_depth, p->max_depth) + 1;
-    if(nrc_on && (!ctx->nrc.params.train || ctx->nrc.params.train_depth > 0))
-    {
-        // the cache ends rendered paths at its query depth and training paths
-        // at theirs
-        const int32_t tail = ctx->nrc.params.train ? ctx->nrc.params.train_depth : 0;
-        bounces = std::min<int64_t>(bounces, (int64_t)std::max(ctx->nrc.params.query_depth, tail) + 1);
-    }
     const bool one_block = ctx->tuning.graph_bounces == 0 && total <= (uint64_t)p->state_count &&
                            bounces <= ONE_BLOCK_BOUNCES && (rows.samples == 0 || rows.samples == p->spp);
     const int check_every = one_block ? (int)bounces : ctx->tuning.graph_bounces > 0 ? ctx->tuning.graph_bounces : 4;

@@ -211,10 +211,12 @@ struct RenderConsts
     int32_t nrc_stride, nrc_phase, nrc_max_paths;
     FilterConsts filter;
     // sample rows of the frame (SAMPLER_HALTON_ROWS): row r holds dimensions 2,
-    // 3, ... of the Halton index of sample row_sample + r / ROW_CELLS at the
-    // pixels whose coordinates modulo 128 are r % ROW_CELLS
+    // 3, ... of a Halton index; rows go through row_width x row_height pixels
+    // (the film's size, at most MAX_HALTON_RESOLUTION each), then the samples
+    // from row_sample on
     const float *rows;
     int32_t row_dims;       // floats per row, a multiple of four
+    int32_t row_width, row_height;
     int32_t row_sample;
     uint64_t total;         // paths to generate (of the frame, or to the end of the rows' samples)
     HaltonTables halton;    // dimensions and first-digit tables of the Halton sampler
@@ -223,12 +225,10 @@ struct RenderConsts
 // A Halton index depends on the pixel only through its coordinates modulo
 // MAX_HALTON_RESOLUTION, so the pixels of a large film share their numbers:
 // 126 of a 1080p film's pixels use each. Row of pixel (px, py) and sample.
-constexpr int32_t ROW_CELLS = MAX_HALTON_RESOLUTION * MAX_HALTON_RESOLUTION;
-
 __device__ __forceinline__ uint32_t sample_row(const RenderConsts &rc, uint32_t px, uint32_t py, int32_t sample)
 {
-    return (uint32_t)(sample - rc.row_sample) * (uint32_t)ROW_CELLS +
-           (py % (uint32_t)MAX_HALTON_RESOLUTION) * (uint32_t)MAX_HALTON_RESOLUTION + px % (uint32_t)MAX_HALTON_RESOLUTION;
+    return ((uint32_t)(sample - rc.row_sample) * (uint32_t)rc.row_height + py % (uint32_t)MAX_HALTON_RESOLUTION) *
+               (uint32_t)rc.row_width + px % (uint32_t)MAX_HALTON_RESOLUTION;
 }
 
 // A pointer loaded from a device-memory record, known to be global: without
@@ -278,9 +278,9 @@ enum : int
 // parity: the bounce's parity (the pool side it reads)
 // before the bounce of this parity (first: no bounce came before it)
 void launch_turn(hipStream_t s, const RenderConsts *rc, WaveCounters *c, int32_t state_count, int parity, bool first);
-// fills `samples` * ROW_CELLS sample rows from first sample `sample` on
-void launch_sample_rows(hipStream_t s, const HaltonConsts &hc, const HaltonTables &tab, int32_t sample, int32_t samples,
-                        int32_t dims, float *rows);
+// fills the sample rows of `samples` samples from `sample` on, width * height each
+void launch_sample_rows(hipStream_t s, const HaltonConsts &hc, const HaltonTables &tab, int32_t width, int32_t height,
+                        int32_t sample, int32_t samples, int32_t dims, float *rows);
 void launch_generate(hipStream_t s, int grid, int sampler, const RenderConsts *rc, const WaveCounters *c,
                      PathSOA path);
 void launch_trace_extension(hipStream_t s, int grid, int sched, const TraceScene &ts, WaveCounters *c,

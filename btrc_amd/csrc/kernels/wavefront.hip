@@ -349,15 +349,14 @@ __global__ void __launch_bounds__(64) k_turn(const RenderConsts *rc, WaveCounter
 // replace the 1.2 million dimensions drawn per sample at the stages.
 constexpr int ROW_TILE = 32;
 
-__global__ void __launch_bounds__(256) k_sample_rows(HaltonConsts hc, HaltonTables tab, int32_t sample, int32_t dims,
-                                                     float *rows)
+__global__ void __launch_bounds__(256) k_sample_rows(HaltonConsts hc, HaltonTables tab, uint32_t width, uint32_t cells,
+                                                     int32_t sample, uint32_t count, int32_t dims, float *rows)
 {
     __shared__ float tile[64][ROW_TILE + 1];
     const uint32_t lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
-    const uint32_t row0 = blockIdx.x * 64; // ROW_CELLS is a multiple of 64: one sample, one pixel row
-    const uint32_t cell = row0 % ROW_CELLS + lane;
-    const HaltonState st = halton_start(hc, cell % MAX_HALTON_RESOLUTION, cell / MAX_HALTON_RESOLUTION,
-                                        sample + (int32_t)(row0 / ROW_CELLS));
+    const uint32_t row0 = blockIdx.x * 64, row = row0 + lane;
+    const uint32_t cell = row % cells;
+    const HaltonState st = halton_start(hc, cell % width, cell / width, sample + (int32_t)(row / cells));
     const uint32_t d0 = blockIdx.y * ROW_TILE;
     for(uint32_t k = 0; k < ROW_TILE / 4; ++k)
     {
@@ -369,7 +368,7 @@ __global__ void __launch_bounds__(256) k_sample_rows(HaltonConsts hc, HaltonTabl
     for(uint32_t t = threadIdx.x; t < 64 * ROW_TILE / 4; t += 256)
     {
         const uint32_t r = t / (ROW_TILE / 4), d = t % (ROW_TILE / 4) * 4;
-        if(d0 + d < (uint32_t)dims)
+        if(d0 + d < (uint32_t)dims && row0 + r < count)
             *reinterpret_cast<float4 *>(rows + (size_t)(row0 + r) * (uint32_t)dims + d0 + d) =
                 make_float4(tile[r][d], tile[r][d + 1], tile[r][d + 2], tile[r][d + 3]);
     }
@@ -1803,11 +1802,12 @@ void launch_halton_eval(hipStream_t s, const HaltonConsts &hc, const HaltonTable
                        out);
 }
 
-void launch_sample_rows(hipStream_t s, const HaltonConsts &hc, const HaltonTables &tab, int32_t sample, int32_t samples,
-                        int32_t dims, float *rows)
+void launch_sample_rows(hipStream_t s, const HaltonConsts &hc, const HaltonTables &tab, int32_t width, int32_t height,
+                        int32_t sample, int32_t samples, int32_t dims, float *rows)
 {
-    hipLaunchKernelGGL(k_sample_rows, dim3(samples * (ROW_CELLS / 64), (dims + ROW_TILE - 1) / ROW_TILE), dim3(256), 0,
-                       s, hc, tab, sample, dims, rows);
+    const uint32_t cells = (uint32_t)(width * height), count = cells * (uint32_t)samples;
+    hipLaunchKernelGGL(k_sample_rows, dim3((count + 63) / 64, (dims + ROW_TILE - 1) / ROW_TILE), dim3(256), 0, s, hc,
+                       tab, (uint32_t)width, cells, sample, count, dims, rows);
 }
 
 void launch_make_bricks(hipStream_t s, const float *grid, int32_t nx, int32_t ny, int32_t nz, uint64_t bricks,

@@ -14,28 +14,30 @@ from util import render_params
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("w,h,min_depth,max_depth,filt", [
-    (512, 384, 3, 8, "box"),          # 12 pixels a row: the first size with rows
-    (512, 383, 3, 8, "box"),          # just below
-    (2048, 128, 0, 3, "gaussian"),
-    (4096, 127, 3, 5, "box"),         # another stride: no rows
-    (640, 400, 9, 2, "gaussian"),     # nine vertices without roulette, then the end
+@pytest.mark.parametrize("w,h,spp,min_depth,max_depth,filt", [
+    (512, 384, 2, 3, 8, "box"),          # 12 pixels a row: the first size with rows
+    (512, 383, 2, 3, 8, "box"),          # just below
+    (2048, 128, 1, 0, 3, "gaussian"),
+    (4096, 127, 1, 3, 5, "box"),         # rows of 128 x 127 pixels, another stride
+    (100, 64, 3, 3, 8, "box"), (129, 33, 1, 2, 6, "gaussian"), (1, 30, 2, 3, 4, "box"),
+    (640, 400, 1, 9, 2, "gaussian"),     # nine vertices without roulette, then the end
 ])
-def test_rows_match_oracle(ctx, w, h, min_depth, max_depth, filt):
+def test_rows_match_oracle(ctx, w, h, spp, min_depth, max_depth, filt):
     scene, cam = scenes.cornell()
     ctx.upload_scene(scene)
     ctx.set_camera(cam, w, h)
     ctx.set_filter(filt)
-    p = render_params(w, h, 1, min_depth=min_depth, max_depth=max_depth, state_count=1 << 18)
+    p = render_params(w, h, spp, min_depth=min_depth, max_depth=max_depth, state_count=1 << 18)
     st = ctx.render(p)
     got = ctx.film(w, h)[0][..., :3].astype(np.float64)
     ctx.set_filter("box")
-    r0, r1 = h // 2, h // 2 + 24
-    ref = oracle.OracleScene(scene).render(cam, p, first=r0 * w, count=(r1 - r0) * w,
-                                           filt=None if filt == "box" else ("gaussian", 1.3, 1.6))[0][r0:r1]
+    r0, r1 = h // 2, min(h, h // 2 + 24)
+    o = oracle.OracleScene(scene)
+    ref = sum(o.render(cam, p, first=(s * h + r0) * w, count=(r1 - r0) * w,
+                       filt=None if filt == "box" else ("gaussian", 1.3, 1.6))[0][r0:r1] for s in range(spp)) / spp
     rel = np.abs(got[r0:r1] - ref) / np.maximum(np.abs(ref), 1e-2)
     assert rel.max() <= 1e-4 and ref.max() > 0
-    assert st.paths == w * h
+    assert st.paths == w * h * spp
 
 
 def fp64_film(ctx, w, h, spp, offset=0, accumulate=0, tile=0, state_count=1 << 20):
