@@ -10,6 +10,8 @@
 #include <new>
 #include <stdexcept>
 #include <string>
+#include <system_error>
+#include <thread>
 #include <vector>
 
 #include "../../../include/btrc_hip.h"
@@ -145,6 +147,50 @@ struct DevBuf
         alloc(n);
         if(n)
             BTRC_HIP_CHECK(hipMemcpyAsync(ptr, src, n * sizeof(T), hipMemcpyHostToDevice, s));
+    }
+};
+
+// Pinned chunks that large results pass through on their way to the caller's
+// pageable memory (read_back), kept with the context: 16 MiB.
+struct ReadRing
+{
+    static constexpr size_t SLOTS = 8, CHUNK = (size_t)1 << 21;
+    unsigned char *mem = nullptr;
+    hipEvent_t ready[SLOTS] = {};
+
+    ReadRing() = default;
+    ReadRing(const ReadRing &) = delete;
+    ReadRing &operator=(const ReadRing &) = delete;
+    ~ReadRing() { release(); }
+
+    void release()
+    {
+        if(mem)
+            (void)hipHostFree(mem);
+        mem = nullptr;
+        for(hipEvent_t &e : ready)
+        {
+            if(e)
+                (void)hipEventDestroy(e);
+            e = nullptr;
+        }
+    }
+    // false: no pinned memory to be had
+    bool init()
+    {
+        if(mem)
+            return true;
+        bool ok = true;
+        for(hipEvent_t &e : ready)
+            ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
+        ok = ok && hipHostMalloc((void **)&mem, SLOTS * CHUNK, hipHostMallocDefault) == hipSuccess;
+        if(!ok)
+        {
+            mem = nullptr;
+            release();
+            (void)hipGetLastError();
+        }
+        return ok;
     }
 };
 
@@ -312,6 +358,7 @@ struct btrc_ctx
     DevBuf<WaveState> counters;       // the counters (read back) and the queue bookkeeping
     WaveCounters *wc() const { return &counters.ptr->c; }
     WaveCounters *host_counters = nullptr; // pinned
+    ReadRing read_ring;
     DevBuf<float> film;
     DevBuf<double> film64;
     DevBuf<float> film_albedo, film_normal;
@@ -484,6 +531,108 @@ int guarded(btrc_ctx *ctx, F &&f)
         ctx->last_error = e.what();
         return BTRC_ERR_INVALID;
     }
+}
+
+// Copies a result of the context's stream to the caller's memory and waits
+// for it; with `scale`, doubles times that. Into pageable memory the runtime
+// copies one staged chunk at a time, and its one thread also takes the page
+// faults of a fresh array. Here chunks stream into the pinned ring while
+// READ_WORKERS threads empty it; chunk i goes through slot i % SLOTS, and the
+// worker that emptied a slot queues its next chunk, so no slot is touched by
+// two workers. A 1003x565 frame with all its outputs (41 MB): 7.51 ms with the
+// runtime's copies, 6.87 with one thread, 6.28 with two and with four, 6.44
+// with eight; chunks of 512 KiB 6.92, 1 MiB 6.27, 2 MiB 6.19, 4 MiB 6.33. Single
+// chunks, and memory that the device reaches by itself, are copied directly.
+constexpr size_t READ_DIRECT = ReadRing::CHUNK;
+constexpr size_t READ_WORKERS = 2;
+static_assert(ReadRing::SLOTS % READ_WORKERS == 0, "each slot belongs to one worker");
+
+bool pageable(const void *p)
+{
+    hipPointerAttribute_t a{};
+    if(hipPointerGetAttributes(&a, p) != hipSuccess)
+    {
+        (void)hipGetLastError();
+        return true;
+    }
+    return a.type == hipMemoryTypeUnregistered;
+}
+
+void read_back(btrc_ctx *ctx, void *dst, const void *src, size_t bytes, double scale = 1.0)
+{
+    hipStream_t s = ctx->stream;
+    auto put = [scale](unsigned char *to, const unsigned char *from, size_t n) {
+        if(scale == 1.0)
+            std::memcpy(to, from, n);
+        else
+            for(size_t k = 0; k < n; k += sizeof(double))
+            {
+                double v;
+                std::memcpy(&v, from + k, sizeof(v));
+                v *= scale;
+                std::memcpy(to + k, &v, sizeof(v));
+            }
+    };
+    unsigned char *out = static_cast<unsigned char *>(dst);
+    const unsigned char *in = static_cast<const unsigned char *>(src);
+    ReadRing &ring = ctx->read_ring;
+    if(bytes <= READ_DIRECT || !pageable(dst) || !ring.init())
+    {
+        BTRC_HIP_CHECK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s));
+        BTRC_HIP_CHECK(hipStreamSynchronize(s));
+        if(scale != 1.0)
+            put(out, out, bytes);
+        return;
+    }
+    constexpr size_t CHUNK = ReadRing::CHUNK, SLOTS = ReadRing::SLOTS;
+    const size_t chunks = (bytes + CHUNK - 1) / CHUNK;
+    auto size_of = [&](size_t i) { return std::min(CHUNK, bytes - i * CHUNK); };
+    auto queue = [&](size_t i) {
+        const size_t slot = i % SLOTS;
+        const hipError_t e = hipMemcpyAsync(ring.mem + slot * CHUNK, in + i * CHUNK, size_of(i), hipMemcpyDeviceToHost, s);
+        return e == hipSuccess ? hipEventRecord(ring.ready[slot], s) : e;
+    };
+    hipError_t err[READ_WORKERS] = {};
+    for(size_t i = 0; i < std::min(chunks, SLOTS) && err[0] == hipSuccess; ++i)
+        err[0] = queue(i);
+    auto drain = [&](size_t w) {
+        hipError_t e = hipSetDevice(ctx->device);
+        for(size_t i = w; i < chunks && e == hipSuccess; i += READ_WORKERS)
+        {
+            e = hipEventSynchronize(ring.ready[i % SLOTS]);
+            if(e != hipSuccess)
+                break;
+            put(out + i * CHUNK, ring.mem + i % SLOTS * CHUNK, size_of(i));
+            if(i + SLOTS < chunks)
+                e = queue(i + SLOTS);
+        }
+        err[w] = e;
+    };
+    if(err[0] == hipSuccess)
+    {
+        std::thread threads[READ_WORKERS];
+        size_t started = 1;
+        try
+        {
+            for(; started < std::min(READ_WORKERS, chunks); ++started)
+                threads[started] = std::thread(drain, started);
+        }
+        catch(const std::system_error &)
+        {
+            // no more threads to be had: this one does their share
+        }
+        drain(0);
+        for(size_t w = started; w < READ_WORKERS; ++w)
+            drain(w);
+        for(size_t w = 1; w < started; ++w)
+            threads[w].join();
+    }
+    for(hipError_t e : err)
+        if(e != hipSuccess)
+        {
+            (void)hipStreamSynchronize(s); // nothing writes the ring any more
+            BTRC_HIP_CHECK(e);
+        }
 }
 
 // AliasTable::initialize (utils/math/alias.cpp:13-58). The sum runs in index
@@ -2398,20 +2547,13 @@ void film_readback(btrc_ctx *ctx, float *rgba, double *rgb64)
         ctx->resolved.alloc(pixels);
         launch_resolve(s, RESOLVE_COLOR, ctx->film.ptr, pixels, 1.0f / (float)ctx->film_spp, ctx->resolved.ptr);
         BTRC_HIP_CHECK(hipGetLastError());
-        BTRC_HIP_CHECK(hipMemcpyAsync(rgba, ctx->resolved.ptr, pixels * sizeof(float4), hipMemcpyDeviceToHost, s));
+        read_back(ctx, rgba, ctx->resolved.ptr, pixels * sizeof(float4));
     }
     if(rgb64)
     {
         if(!ctx->film_has64)
             throw StateError("the last render had no FP64 film");
-        BTRC_HIP_CHECK(hipMemcpyAsync(rgb64, ctx->film64.ptr, 3 * (size_t)pixels * sizeof(double), hipMemcpyDeviceToHost, s));
-    }
-    BTRC_HIP_CHECK(hipStreamSynchronize(s));
-    if(rgb64)
-    {
-        const double inv = 1.0 / (double)ctx->film_spp;
-        for(size_t i = 0; i < 3 * (size_t)pixels; ++i)
-            rgb64[i] *= inv;
+        read_back(ctx, rgb64, ctx->film64.ptr, 3 * (size_t)pixels * sizeof(double), 1.0 / (double)ctx->film_spp);
     }
 }
 
@@ -2432,8 +2574,7 @@ void tonemap_readback(btrc_ctx *ctx, float exposure, float *rgba)
     BTRC_HIP_CHECK(hipGetLastError());
     launch_tonemap_aces(s, ctx->resolved.ptr, pixels, exposure);
     BTRC_HIP_CHECK(hipGetLastError());
-    BTRC_HIP_CHECK(hipMemcpyAsync(rgba, ctx->resolved.ptr, pixels * sizeof(float4), hipMemcpyDeviceToHost, s));
-    BTRC_HIP_CHECK(hipStreamSynchronize(s));
+    read_back(ctx, rgba, ctx->resolved.ptr, pixels * sizeof(float4));
 }
 
 // preview.cpp generate_albedo / generate_normal
@@ -2451,15 +2592,13 @@ void aov_readback(btrc_ctx *ctx, float *albedo, float *normal)
     {
         launch_resolve(s, RESOLVE_COLOR, ctx->film_albedo.ptr, pixels, inv, ctx->resolved.ptr);
         BTRC_HIP_CHECK(hipGetLastError());
-        BTRC_HIP_CHECK(hipMemcpyAsync(albedo, ctx->resolved.ptr, pixels * sizeof(float4), hipMemcpyDeviceToHost, s));
-        BTRC_HIP_CHECK(hipStreamSynchronize(s));
+        read_back(ctx, albedo, ctx->resolved.ptr, pixels * sizeof(float4));
     }
     if(normal)
     {
         launch_resolve(s, RESOLVE_NORMAL, ctx->film_normal.ptr, pixels, inv, ctx->resolved.ptr);
         BTRC_HIP_CHECK(hipGetLastError());
-        BTRC_HIP_CHECK(hipMemcpyAsync(normal, ctx->resolved.ptr, pixels * sizeof(float4), hipMemcpyDeviceToHost, s));
-        BTRC_HIP_CHECK(hipStreamSynchronize(s));
+        read_back(ctx, normal, ctx->resolved.ptr, pixels * sizeof(float4));
     }
 }
 
@@ -2760,8 +2899,7 @@ int btrc_hip_view_readback(btrc_ctx *ctx, int32_t view, float *rgba)
         launch_resolve(s, RESOLVE_COLOR, ctx->film.ptr + 4 * (size_t)v.pixel_base, pixels,
                        1.0f / (float)ctx->film_spp, ctx->resolved.ptr);
         BTRC_HIP_CHECK(hipGetLastError());
-        BTRC_HIP_CHECK(hipMemcpyAsync(rgba, ctx->resolved.ptr, pixels * sizeof(float4), hipMemcpyDeviceToHost, s));
-        BTRC_HIP_CHECK(hipStreamSynchronize(s));
+        read_back(ctx, rgba, ctx->resolved.ptr, pixels * sizeof(float4));
     });
 }
 
