@@ -3020,37 +3020,38 @@ int btrc_hip_nrc_eval(btrc_ctx *ctx, const float *vertices, int32_t n, float *ou
         nrc_sync(ctx);
         if(n == 0)
             return;
-        DevBuf<NrcVertex> dv;
-        DevBuf<float> dout;
-        dv.upload(reinterpret_cast<const NrcVertex *>(vertices), n, ctx->stream);
-        dout.alloc(3 * (size_t)n);
-        launch_nrc_eval(ctx->stream, nrc_weights(ctx), nrc_box(ctx), dv.ptr, n, dout.ptr);
+        // queries and answers in the layer-input scratch, idle outside
+        // training, where they fit (661,000 queries); allocating and freeing
+        // them is slower than the kernel
+        const size_t in = (size_t)n * sizeof(NrcVertex), bytes = in + 3 * (size_t)n * sizeof(float);
+        DevBuf<uint16_t> own;
+        DevBuf<uint16_t> &buf = bytes <= ctx->nrc.xt.count * sizeof(uint16_t) ? ctx->nrc.xt : own;
+        if(&buf == &own)
+            own.alloc(bytes / sizeof(uint16_t));
+        NrcVertex *dv = reinterpret_cast<NrcVertex *>(buf.ptr);
+        float *dout = reinterpret_cast<float *>(dv + n);
+        BTRC_HIP_CHECK(hipMemcpyAsync(dv, vertices, in, hipMemcpyHostToDevice, ctx->stream));
+        launch_nrc_eval(ctx->stream, nrc_weights(ctx), nrc_box(ctx), dv, n, dout);
         BTRC_HIP_CHECK(hipGetLastError());
-        BTRC_HIP_CHECK(hipMemcpyAsync(out, dout.ptr, 3 * (size_t)n * sizeof(float), hipMemcpyDeviceToHost, ctx->stream));
+        BTRC_HIP_CHECK(hipMemcpyAsync(out, dout, bytes - in, hipMemcpyDeviceToHost, ctx->stream));
         BTRC_HIP_CHECK(hipStreamSynchronize(ctx->stream));
     });
 }
 
-// records whose target is `targets`: throughput 1, nothing gathered before,
-// one training path per record carrying the target as its radiance sum
+// `n` vertices and their targets as a training batch (k_nrc_load). The inputs
+// pass through the layer-input scratch, which the training kernels write later
+// on the same stream.
 void nrc_load_batch(btrc_ctx *ctx, const float *vertices, const float *targets, int32_t n)
 {
     auto &nc = ctx->nrc;
-    std::vector<NrcRecord> rec(NRC_RECORDS);
-    std::vector<float> acc(4 * (size_t)NRC_RECORDS, 0.0f);
-    for(int32_t i = 0; i < n; ++i)
-    {
-        NrcRecord &r = rec[i];
-        std::memcpy(&r.v, vertices + 16 * (size_t)i, sizeof(NrcVertex));
-        r.beta[0] = r.beta[1] = r.beta[2] = 1.0f;
-        r.gathered[0] = r.gathered[1] = r.gathered[2] = 0.0f;
-        r.path = (uint32_t)i;
-        r.valid = 1;
-        for(int c = 0; c < 3; ++c)
-            acc[4 * (size_t)i + c] = targets[3 * (size_t)i + c];
-    }
-    nc.rec[0].upload(rec.data(), rec.size(), ctx->stream);
-    nc.acc[0].upload(acc.data(), acc.size(), ctx->stream);
+    static_assert(sizeof(NrcVertex) == 16 * sizeof(float), "a vertex is a row of the caller's array");
+    static_assert((16 + 3) * sizeof(float) <= NRC_LAYERS * NRC_IN * sizeof(uint16_t), "both inputs fit the scratch");
+    NrcVertex *dv = reinterpret_cast<NrcVertex *>(nc.xt.ptr);
+    float *dt = reinterpret_cast<float *>(dv + n);
+    BTRC_HIP_CHECK(hipMemcpyAsync(dv, vertices, (size_t)n * sizeof(NrcVertex), hipMemcpyHostToDevice, ctx->stream));
+    BTRC_HIP_CHECK(hipMemcpyAsync(dt, targets, 3 * (size_t)n * sizeof(float), hipMemcpyHostToDevice, ctx->stream));
+    launch_nrc_load(ctx->stream, nc.rec[0].ptr, nc.acc[0].ptr, dv, dt, n);
+    BTRC_HIP_CHECK(hipGetLastError());
 }
 
 int btrc_hip_nrc_gradients(btrc_ctx *ctx, const float *vertices, const float *targets, int32_t n, float *grad,

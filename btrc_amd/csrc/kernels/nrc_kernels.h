@@ -143,6 +143,9 @@ void launch_nrc_train_step(hipStream_t s, const NrcWeights &net, const NrcBox &b
 void launch_nrc_gradients(hipStream_t s, const NrcWeights &net, const NrcBox &box, const NrcBatch &b,
                           const NrcScratch &sc, float *grad);
 void launch_nrc_clear(hipStream_t s, NrcRecord *rec, int64_t nrec, float *acc, int64_t npaths);
+// rec[0, 2^16) and the rows of acc = n vertices with their targets, then empty
+void launch_nrc_load(hipStream_t s, NrcRecord *rec, float *acc, const NrcVertex *vertices, const float *targets,
+                     int32_t n);
 // index = the valid record slots among rec[0, 2^16) in the order of
 // nrc_record_slot(0, 1, ...), *total = how many (deterministic); mask: 1024
 // words of scratch
