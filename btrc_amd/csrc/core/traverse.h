@@ -44,39 +44,51 @@ static_assert(sizeof(BvhNode4) == 128, "BvhNode4 must be one 128-byte line");
 // multiply-add b * inv + c, with the rounding of c paid for in advance.
 struct RayBoxPre
 {
-    V3 inv;   // 1 / d, at most 2^96 in magnitude
+    V3 inv;   // 1 / d, bounded (raybox_axis)
     V3 near_c; // -o / d, lowered: entry distances never come out late
     V3 far_c;  // -o / d, raised: exit distances never come out early
     bool neg_x, neg_y, neg_z;
 };
 
-// One axis. With inv = 1/d (1 + e1) and oi = o inv (1 + e2), |e| <= 2^-24,
-// the plane distance fma(b, inv, -oi) differs from (b - o) / d by at most
+// One axis, inv = |1 / d|. With v = 1/d (1 + e1) and oi = o v (1 + e2), |e| <=
+// 2^-24, the plane distance fma(b, v, -oi) differs from (b - o) / d by at most
 // 2^-23 of itself plus 2^-24 |oi|. near_c and far_c move by 2^-22 |oi| (and
 // their own rounding takes at most 2^-24 of it), so only the relative part is
-// left, which raybox_nf pays on the exit side. Directions of magnitude below
-// 2^-96 (zero among them) count as 2^-96: their planes lie beyond every
-// scene, and the 2^-80 |inv| term keeps a ray that runs inside a plane of the
-// box (o on it, d zero) inside the box.
-BTRC_HD void raybox_axis(float o, float d, float *inv, float *near_c, float *far_c)
+// left, which raybox_nf pays on the exit side.
+//
+// An axis on which the ray hardly moves (zero directions among them) counts as
+// inv = `big`, which keeps o v finite for every origin. That pulls its planes
+// towards the origin: a plane behind an origin outside the slab stays behind
+// it, and the planes around an origin inside, or on one of them, move out by
+// `reach`, which no hit's distance exceeds.
+BTRC_HD void raybox_axis(float o, float d, float inv, float big, float reach, float *v_out, float *near_c, float *far_c)
 {
-    const float big = 7.9228163e28f; // 2^96
-    const float m = fmaxf(fminf(fabsf(1.0f / d), big), 1.1754944e-38f); // never 0: an empty slot's planes stay infinite
+    const float m = fmaxf(fminf(inv, big), 2.9387359e-39f); // 2^-128, never 0: an empty slot's planes stay infinite
     const float v = u2f(f2u(m) | (f2u(d) & 0x80000000u));
     const float oi = o * v;
     const float up = 1.0f + 2.3841858e-7f, down = 1.0f - 2.3841858e-7f; // 1 +- 2^-22
-    const float tiny = m * 8.2718061e-25f;                              // 2^-80 |inv|
-    *inv = v;
-    *near_c = -(oi * (oi > 0.0f ? up : down)) - tiny;
-    *far_c = -(oi * (oi > 0.0f ? down : up)) + tiny;
+    const float out = inv > big ? reach : 0.0f;
+    *v_out = v;
+    *near_c = -(oi * (oi > 0.0f ? up : down)) - out;
+    *far_c = -(oi * (oi > 0.0f ? down : up)) + out;
 }
 
 BTRC_HD RayBoxPre raybox_pre(V3 o, V3 d)
 {
     RayBoxPre p;
-    raybox_axis(o.x, d.x, &p.inv.x, &p.near_c.x, &p.far_c.x);
-    raybox_axis(o.y, d.y, &p.inv.y, &p.near_c.y, &p.far_c.y);
-    raybox_axis(o.z, d.z, &p.inv.z, &p.near_c.z, &p.far_c.z);
+    const float ix = fabsf(1.0f / d.x), iy = fabsf(1.0f / d.y), iz = fabsf(1.0f / d.z);
+    // big = 2^120 / max(|o|, 1) to a power of two: |o| big < 2^121
+    const float mo = fmaxf(fmaxf(fabsf(o.x), fabsf(o.y)), fmaxf(fabsf(o.z), 1.0f));
+    const float big = u2f((374u << 23) - (f2u(mo) & 0x7f800000u));
+    // A hit lies within 2^64 units (beyond them the triangle tests overflow),
+    // so at t below 2^64 / the largest |d|, or at no finite t; no |d| at all:
+    // no hit. The planes of a bounded axis thus move by 2^-56 max(|o|, 1) units
+    // for a ray of unit length, more for shorter ones.
+    const float slow = fminf(ix, fminf(iy, iz)); // 1 / the largest |d|
+    const float reach = slow <= MAX_FLOAT ? fminf(slow * 1.8446744e19f, MAX_FLOAT) : 0.0f;
+    raybox_axis(o.x, d.x, ix, big, reach, &p.inv.x, &p.near_c.x, &p.far_c.x);
+    raybox_axis(o.y, d.y, iy, big, reach, &p.inv.y, &p.near_c.y, &p.far_c.y);
+    raybox_axis(o.z, d.z, iz, big, reach, &p.inv.z, &p.near_c.z, &p.far_c.z);
     p.neg_x = (f2u(d.x) >> 31) != 0;
     p.neg_y = (f2u(d.y) >> 31) != 0;
     p.neg_z = (f2u(d.z) >> 31) != 0;

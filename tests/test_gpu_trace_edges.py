@@ -15,9 +15,9 @@ from util import assert_hits_equal, random_rays
 pytestmark = pytest.mark.gpu
 
 
-def lattice_scene(accel):
+def lattice_scene(accel, scale=1.0):
     """axis-aligned quads on integer planes (flat boxes, shared edges,
-    coplanar duplicates) and a displaced sphere"""
+    coplanar duplicates) and a displaced sphere, `scale` times as large"""
     tris = []
     for k in range(4):
         for i in range(3):
@@ -25,12 +25,13 @@ def lattice_scene(accel):
                 tris.append(scenes.quad((i, j, k), (i + 1, j, k), (i + 1, j + 1, k), (i, j + 1, k)))
                 tris.append(scenes.quad((k, i, j), (k, i + 1, j), (k, i + 1, j + 1), (k, i, j + 1)))
                 tris.append(scenes.quad((i, k, j), (i, k, j + 1), (i + 1, k, j + 1), (i + 1, k, j)))
-    tris = np.concatenate(tris).reshape(-1, 9)
+    tris = np.concatenate(tris).reshape(-1, 9) * np.float32(scale)
+    ball = scenes.uv_sphere(scenes.PCG32(4), displacement=0.2) * np.float32(scale)
     s = scenes.Scene()
     m = s.add_diffuse([0.5, 0.5, 0.5])
     s.add_instance(s.add_geometry(tris), m)
     s.add_instance(s.add_geometry(tris[::3].copy()), m)          # ties
-    s.add_instance(s.add_geometry(scenes.uv_sphere(scenes.PCG32(4), displacement=0.2)), m, np.eye(4))
+    s.add_instance(s.add_geometry(ball), m, np.eye(4))
     s.accel = accel
     return s
 
@@ -74,6 +75,38 @@ def test_edge_rays_equal_brute_force(ctx, accel, mode):
         same = (got["instance"] == want["instance"]) & (got["prim"] == want["prim"])
         assert same.mean() > 0.99
     assert np.array_equal(ctx.trace_any(rays, mode), ref.trace(rays, mode, any_hit=True, use_bvh=False))
+
+
+@pytest.mark.parametrize("accel", [_abi.ACCEL_FLAT, _abi.ACCEL_TWO_LEVEL])
+@pytest.mark.parametrize("scale,length", [(2.0 ** 20, 1.0), (2.0 ** 31, 1.0), (1.0, 2.0 ** -60), (1.0, 2.0 ** -97),
+                                          (2.0 ** -20, 2.0 ** -110), (1.0, 2.0 ** 60)])
+def test_any_magnitude_equals_brute_force(ctx, accel, scale, length):
+    """scenes of large extent (origins beyond 2^32, rays that run inside a
+    box's face for millions of units) and rays far from unit length; zero,
+    negative-zero and very small components among the directions"""
+    scene = lattice_scene(accel, scale)
+    ctx.upload_scene(scene)
+    rng = np.random.default_rng(17)
+    n = 6000
+    rays = np.zeros(n, dtype=_abi.ray_dtype())
+    rays["o"] = rng.integers(-2, 10, (n, 3)).astype(np.float32) * np.float32(0.5 * scale)
+    d = rng.choice([0.0, -0.0, 1.0, -1.0, 0.5, 2.0 ** -25, 3.0], (n, 3)).astype(np.float32)
+    d[(d == 0).all(axis=1), 0] = 1.0
+    rays["d"] = d * np.float32(length)
+    rays["tmax"] = np.float32(3.4028234663852886e38)
+    ref = oracle.OracleScene(scene)
+    got, want = ctx.trace_closest(rays), ref.trace(rays, use_bvh=False)
+    assert 0.1 < (want["instance"] != 0xffffffff).mean() < 0.95
+    if length == 1.0:
+        assert_hits_equal(got, want)
+    else:
+        # the culling margin is a distance along a ray of unit length: a
+        # shorter ray may keep the other of two hits a few roundings (2^-24 of
+        # a vertex' distance, up to 6 units) apart
+        assert np.array_equal(got["instance"] == 0xffffffff, want["instance"] == 0xffffffff)
+        np.testing.assert_allclose(got["t"].astype(np.float64) * length, want["t"].astype(np.float64) * length,
+                                   rtol=4 * 2.0 ** -24, atol=4 * 6 * scale * 2.0 ** -24)
+    assert np.array_equal(ctx.trace_any(rays), ref.trace(rays, any_hit=True, use_bvh=False))
 
 
 @pytest.mark.parametrize("n", [1, 63, 64, 65, 1000, 24 * 256 * 64 + 1])
