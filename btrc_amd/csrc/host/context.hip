@@ -1976,6 +1976,9 @@ constexpr int64_t ROWS_MIN_SHARE = 12;
 constexpr int64_t ROWS_SMALL_VALUES = 2 << 20;
 constexpr size_t ROWS_MAX_BYTES = (size_t)2 << 30;
 
+// paths in flight that fill the GPU in every launch of a bounce
+constexpr int64_t FULL_BOUNCE = 1 << 20;
+
 struct SampleRows
 {
     int32_t samples = 0, dims = 0, width = 0, height = 0;
@@ -2261,14 +2264,30 @@ void render(btrc_ctx *ctx, const btrc_render_params *p, int32_t view_count, cons
     int64_t captured = 0;
     const auto t0 = std::chrono::steady_clock::now();
     int cur = 0;
-    // Bounces per captured block, even: a block ends on the pool side it began
-    // with. A frame whose paths all fit the pool needs no more than `bounces`:
-    // up to ONE_BLOCK_BOUNCES of them run as one block with one read-back,
-    // generating in the first bounce only.
+    const bool use_graph = ctx->tuning.launch_graph && !timer.enabled && !capture;
+    // Bounces between read-backs, even: a captured block ends on the pool side
+    // it began with. Progress is reported and a stop request seen there.
+    //
+    // A frame whose paths all fit the pool needs no more than `bounces`: up to
+    // ONE_BLOCK_BOUNCES of them (odd numbers too) run as one block with one
+    // read-back, generating in the first bounce only, unless somebody follows
+    // the progress. Only frames that do not fill the GPU: they end within
+    // milliseconds, so a stop request that finds one running waits for its end,
+    // and larger ones gain next to nothing.
     constexpr int ONE_BLOCK_BOUNCES = 10;
-    const bool one_block = ctx->tuning.graph_bounces == 0 && total <= (uint64_t)p->state_count &&
+    const int64_t most_rays = (int64_t)std::min<uint64_t>((uint64_t)p->state_count, total);
+    const bool one_block = use_graph && ctx->tuning.graph_bounces == 0 && !ctx->reporter.progress &&
+                           total <= (uint64_t)p->state_count && most_rays < FULL_BOUNCE &&
                            bounces <= ONE_BLOCK_BOUNCES && (rows.samples == 0 || rows.samples == p->spp);
     const int check_every = one_block ? (int)bounces : ctx->tuning.graph_bounces > 0 ? ctx->tuning.graph_bounces : 4;
+    // (the stream is idle when a stopped render returns: the next one writes
+    // the pinned constants and counters again)
+    auto check_stop = [&] {
+        if(!ctx->stop.load())
+            return;
+        BTRC_HIP_CHECK(hipStreamSynchronize(s));
+        throw Stopped("render stopped");
+    };
 
     // one bounce: generate, trace, [medium], shade, shadow, then the turn to
     // the next. With `overlap` the shadow rays go to the shadow stream and are
@@ -2316,7 +2335,6 @@ void render(btrc_ctx *ctx, const btrc_render_params *p, int32_t view_count, cons
     };
     // a block of bounces whose launches do not fill the GPU: a bounce's shadow
     // rays share a launch with the next bounce's extension rays
-    const int64_t most_rays = (int64_t)std::min<uint64_t>((uint64_t)p->state_count, total);
     auto small_grid = [&](int full) {
         return (int)std::min<int64_t>(std::min(full, ctx->cu_count * TRACE_WAVES_ANY), (most_rays + 63) / 64);
     };
@@ -2343,7 +2361,7 @@ void render(btrc_ctx *ctx, const btrc_render_params *p, int32_t view_count, cons
                       (check_every - 1) & 1);
     };
 
-    if(ctx->tuning.launch_graph && !timer.enabled && !capture)
+    if(use_graph)
     {
         // blocks of check_every bounces from a captured graph; recaptured
         // when any launch argument differs from the cached graph's
@@ -2358,7 +2376,7 @@ void render(btrc_ctx *ctx, const btrc_render_params *p, int32_t view_count, cons
         // the shadow stream pays off once a bounce fills the GPU: the event
         // hand-offs cost ~6 us per bounce (256^2 frames: +8 %), the overlap
         // saves ~7 % of a 1080p frame
-        const bool overlap = most_rays >= (1 << 20);
+        const bool overlap = most_rays >= FULL_BOUNCE;
         // (the joint launch is compiled for the default schedules)
         const bool small = !overlap && !(ctx->trace_sched(false) & SCHED_POSTPONE) && !(ctx->trace_sched(true) & SCHED_POSTPONE);
         const int32_t ints[12] = { grid256, ctx->trace_grid, ctx->trace_sched(false), ctx->trace_sched(true),
@@ -2400,11 +2418,12 @@ void render(btrc_ctx *ctx, const btrc_render_params *p, int32_t view_count, cons
         while(next_window())
         for(;;)
         {
-            if(ctx->stop.load())
-                throw Stopped("render stopped");
+            check_stop();
             BTRC_HIP_CHECK(hipGraphLaunch(ctx->loop_exec[g], s));
             BTRC_HIP_CHECK(hipMemcpyAsync(ctx->host_counters, ctx->wc(), sizeof(WaveCounters), hipMemcpyDeviceToHost, s));
             BTRC_HIP_CHECK(hipStreamSynchronize(s));
+            if(one_block)
+                check_stop();
             const WaveCounters &hc = *ctx->host_counters;
             reporter_stage.progress(hc, total);
             if(hc.generated == window_total && hc.active == 0)
@@ -2417,8 +2436,7 @@ void render(btrc_ctx *ctx, const btrc_render_params *p, int32_t view_count, cons
     for(uint64_t iter = 0; next_window();)
     for(;; ++iter)
     {
-        if(ctx->stop.load())
-            throw Stopped("render stopped");
+        check_stop();
         PathSOA path = ctx->pool[cur].view();
         PathSOA next = ctx->pool[cur ^ 1].view();
         timer.run(STAGE_GENERATE, [&] { launch_generate(s, grid256, sampler, rcd, ctx->wc(), path); });

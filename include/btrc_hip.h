@@ -371,8 +371,10 @@ typedef struct btrc_tuning
                                         postpone leaves (default 0: both test leaves when reached) */
     int32_t stage_blocks_per_cu;     /* grid of the 256-lane stage kernels (generate, medium, shade): at most
                                         this many workgroups per CU, 1..64 (0: 32) */
-    int32_t graph_bounces;           /* bounces per captured graph block between counter read-backs,
-                                        even, 2..16 (0: 4) */
+    int32_t graph_bounces;           /* bounces per captured graph block between counter read-backs, where
+                                        progress is reported and a stop request seen; even, 2..16. 0: 4, or
+                                        a whole frame of at most 10 bounces and 2^20 - 1 paths that all fit
+                                        the pool, where no progress callback is set */
     int32_t reserved;
 } btrc_tuning;
 

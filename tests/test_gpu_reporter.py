@@ -65,3 +65,32 @@ def test_reporter_stage_completes_when_stopped(ctx):
         ctx.set_reporter(None)
     assert rec.calls[0][0] == "new_stage" and rec.calls[-1] == ("complete_stage",)
     assert sum(1 for c in rec.calls if c[0] == "progress") == 1
+
+
+@pytest.mark.parametrize("stop", [False, True])
+def test_progress_and_stop_within_a_frame_that_fits_the_pool(ctx, stop):
+    """nine bounces, every path in flight at once: progress comes after each
+    four, and a stop request from the first one ends the render"""
+    scene, cam = scenes.cornell()
+    ctx.upload_scene(scene)
+    ctx.set_camera(cam, 64, 64)
+    p = render_params(64, 64, 4, min_depth=8, max_depth=8, state_count=1 << 14)
+    plain = ctx.render(p)
+    rec = Recorder(stop_ctx=ctx if stop else None)
+    ctx.set_reporter(rec)
+    try:
+        if stop:
+            with pytest.raises(btrc_amd.BtrcException) as e:
+                ctx.render(p)
+            assert e.value.status == _abi.BTRC_ERR_STOPPED
+        else:
+            st = ctx.render(p)
+            assert (st.extension_rays, st.shadow_rays) == (plain.extension_rays, plain.shadow_rays)
+    finally:
+        ctx.set_reporter(None)
+    pct = [c[1] for c in rec.calls if c[0] == "progress"]
+    assert len(pct) == (1 if stop else 3)
+    assert all(0.0 <= a <= b for a, b in zip(pct, pct[1:])) and (stop or pct[-1] == 100.0)
+    # the context renders on as before
+    st = ctx.render(p)
+    assert (st.extension_rays, st.shadow_rays) == (plain.extension_rays, plain.shadow_rays)
