@@ -54,41 +54,38 @@ struct RayBoxPre
 // 2^-24, the plane distance fma(b, v, -oi) differs from (b - o) / d by at most
 // 2^-23 of itself plus 2^-24 |oi|. near_c and far_c move by 2^-22 |oi| (and
 // their own rounding takes at most 2^-24 of it), so only the relative part is
-// left, which raybox_nf pays on the exit side.
-//
-// An axis on which the ray hardly moves (zero directions among them) counts as
-// inv = `big`, which keeps o v finite for every origin. That pulls its planes
-// towards the origin: a plane behind an origin outside the slab stays behind
-// it, and the planes around an origin inside, or on one of them, move out by
-// `reach`, which no hit's distance exceeds.
-BTRC_HD void raybox_axis(float o, float d, float inv, float big, float reach, float *v_out, float *near_c, float *far_c)
+// left, which raybox_nf pays on the exit side; then by the distance along the
+// ray of `out` units on this axis.
+BTRC_HD void raybox_axis(float o, float d, float inv, float big, float out, float *v_out, float *near_c, float *far_c)
 {
     const float m = fmaxf(fminf(inv, big), 2.9387359e-39f); // 2^-128, never 0: an empty slot's planes stay infinite
     const float v = u2f(f2u(m) | (f2u(d) & 0x80000000u));
     const float oi = o * v;
-    const float up = 1.0f + 2.3841858e-7f, down = 1.0f - 2.3841858e-7f; // 1 +- 2^-22
-    const float out = inv > big ? reach : 0.0f;
     *v_out = v;
-    *near_c = -(oi * (oi > 0.0f ? up : down)) - out;
-    *far_c = -(oi * (oi > 0.0f ? down : up)) + out;
+    *near_c = fmaf(m, -out, fmaf(fabsf(oi), -2.3841858e-7f, -oi)); // 2^-22
+    *far_c = fmaf(m, out, fmaf(fabsf(oi), 2.3841858e-7f, -oi));
 }
 
 BTRC_HD RayBoxPre raybox_pre(V3 o, V3 d)
 {
     RayBoxPre p;
     const float ix = fabsf(1.0f / d.x), iy = fabsf(1.0f / d.y), iz = fabsf(1.0f / d.z);
-    // big = 2^120 / max(|o|, 1) to a power of two: |o| big < 2^121
+    // An axis on which the ray hardly moves (zero directions among them)
+    // counts as 1 / |d| = big = 2^120 / max(|o|, 1), to a power of two, which
+    // keeps o v finite for every origin. That pulls its planes towards the
+    // origin: a plane on the other side of it stays there; the planes around an
+    // origin inside the slab, or on one of them, are moved out past every hit
+    // by out = 2^-56 max(|o|, 1) / the largest |d| (out * big exceeds any t
+    // that 2^63 units can take, where the triangle tests overflow). On other
+    // axes that is next to nothing. Without any |d| there is no hit.
     const float mo = fmaxf(fmaxf(fabsf(o.x), fabsf(o.y)), fmaxf(fabsf(o.z), 1.0f));
-    const float big = u2f((374u << 23) - (f2u(mo) & 0x7f800000u));
-    // A hit lies within 2^64 units (beyond them the triangle tests overflow),
-    // so at t below 2^64 / the largest |d|, or at no finite t; no |d| at all:
-    // no hit. The planes of a bounded axis thus move by 2^-56 max(|o|, 1) units
-    // for a ray of unit length, more for shorter ones.
+    const uint32_t exponent = f2u(mo) & 0x7f800000u;
+    const float big = u2f((374u << 23) - exponent);
     const float slow = fminf(ix, fminf(iy, iz)); // 1 / the largest |d|
-    const float reach = slow <= MAX_FLOAT ? fminf(slow * 1.8446744e19f, MAX_FLOAT) : 0.0f;
-    raybox_axis(o.x, d.x, ix, big, reach, &p.inv.x, &p.near_c.x, &p.far_c.x);
-    raybox_axis(o.y, d.y, iy, big, reach, &p.inv.y, &p.near_c.y, &p.far_c.y);
-    raybox_axis(o.z, d.z, iz, big, reach, &p.inv.z, &p.near_c.z, &p.far_c.z);
+    const float out = slow <= MAX_FLOAT ? slow * u2f(exponent - (56u << 23)) : 0.0f;
+    raybox_axis(o.x, d.x, ix, big, out, &p.inv.x, &p.near_c.x, &p.far_c.x);
+    raybox_axis(o.y, d.y, iy, big, out, &p.inv.y, &p.near_c.y, &p.far_c.y);
+    raybox_axis(o.z, d.z, iz, big, out, &p.inv.z, &p.near_c.z, &p.far_c.z);
     p.neg_x = (f2u(d.x) >> 31) != 0;
     p.neg_y = (f2u(d.y) >> 31) != 0;
     p.neg_z = (f2u(d.z) >> 31) != 0;
