@@ -373,8 +373,8 @@ typedef struct btrc_tuning
                                         this many workgroups per CU, 1..64 (0: 32) */
     int32_t graph_bounces;           /* bounces per captured graph block between counter read-backs, where
                                         progress is reported and a stop request seen; even, 2..16. 0: 4, or
-                                        a whole frame of at most 10 bounces and 2^20 - 1 paths that all fit
-                                        the pool, where no progress callback is set */
+                                        without a progress callback a whole frame of at most 10 bounces whose
+                                        paths all fit the pool */
     int32_t reserved;
 } btrc_tuning;
 

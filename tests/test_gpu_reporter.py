@@ -2,6 +2,9 @@
 WavefrontPathTracer::render calls it, wavefront.cpp:221,287,314): one new
 stage, progress rising to 100 % of the frame's paths, one completed stage,
 also when the render is stopped from inside a progress callback."""
+import threading
+import time
+
 import pytest
 
 import btrc_amd
@@ -94,3 +97,31 @@ def test_progress_and_stop_within_a_frame_that_fits_the_pool(ctx, stop):
     # the context renders on as before
     st = ctx.render(p)
     assert (st.extension_rays, st.shadow_rays) == (plain.extension_rays, plain.shadow_rays)
+
+
+def test_stop_request_while_a_frame_that_fits_the_pool_runs(ctx):
+    """without a progress callback such a frame has one read-back; a request
+    from another thread meanwhile still ends it as stopped"""
+    scene, cam = scenes.cornell()
+    ctx.upload_scene(scene)
+    ctx.set_camera(cam, 2048, 2048)
+    p = render_params(2048, 2048, 4, min_depth=8, max_depth=8, state_count=1 << 24)
+    ctx.render(p)
+    t = time.perf_counter()
+    plain = ctx.render(p)
+    seconds = time.perf_counter() - t
+    assert seconds > 0.005
+
+    def stop():
+        time.sleep(0.3 * seconds)
+        ctx.lib.btrc_hip_request_stop(ctx.h)
+
+    th = threading.Thread(target=stop)
+    th.start()
+    try:
+        with pytest.raises(btrc_amd.BtrcException) as e:
+            ctx.render(p)
+        assert e.value.status == _abi.BTRC_ERR_STOPPED
+    finally:
+        th.join()
+    assert ctx.render(p).extension_rays == plain.extension_rays
