@@ -767,6 +767,18 @@ void set_filter(btrc_ctx *ctx, const btrc_filter_desc *f)
     ctx->filter = FilterConsts{ FILTER_GAUSSIAN, r, 2 * r / G, ctx->filter_table.ptr };
 }
 
+// Sample rows (alloc_sample_rows) stay with the context between frames: up to
+// ROWS_KEEP_BYTES whatever is rendered, more only while frames use at least a
+// quarter of them. A scene, a pool or a film about to be allocated comes first.
+constexpr size_t ROWS_KEEP_BYTES = (size_t)64 << 20;
+
+void trim_sample_rows(btrc_ctx *ctx, size_t needed_floats)
+{
+    const size_t held = ctx->sample_rows.count;
+    if(held * sizeof(float) > ROWS_KEEP_BYTES && held / 4 > needed_floats)
+        ctx->sample_rows.release();
+}
+
 // persistent traversal grid and the per-lane stack overflow it needs
 void size_traversal(btrc_ctx *ctx)
 {
@@ -1129,6 +1141,7 @@ void upload_scene(btrc_ctx *ctx, const btrc_scene_desc *sd)
     if((uint32_t)sd->instance_count > PATH_FLAG_INSTANCE_ID_MASK)
         throw InvalidArg("too many instances");
 
+    trim_sample_rows(ctx, 0);
     hipStream_t s = ctx->stream;
 
     // geometries: TriangleMesh::commit per-triangle records (triangle_mesh.cpp:24-171)
@@ -1984,8 +1997,8 @@ struct SampleRows
     int32_t samples = 0, dims = 0, width = 0, height = 0;
 };
 
-SampleRows plan_sample_rows(btrc_ctx *ctx, const btrc_render_params *p, const std::vector<ViewRec> &views,
-                            uint64_t pixels, bool media, int64_t bounces)
+SampleRows plan_sample_rows(const btrc_render_params *p, const std::vector<ViewRec> &views, uint64_t pixels,
+                            bool media, int64_t bounces)
 {
     SampleRows r;
     if(p->sampler != BTRC_SAMPLER_HALTON)
@@ -2006,8 +2019,15 @@ SampleRows plan_sample_rows(btrc_ctx *ctx, const btrc_render_params *p, const st
         return r;
     r.samples = (int32_t)std::min<int64_t>(p->spp, fit);
     r.dims = (int32_t)dims;
+    return r;
+}
+
+// the rows' memory; none to be had: the digit loop, which needs none
+SampleRows alloc_sample_rows(btrc_ctx *ctx, const SampleRows &r)
+{
     // the tracking kernel loads a chunk of a row past its end
-    const size_t floats = (size_t)r.samples * cells * dims + 16;
+    const size_t floats = r.samples > 0 ? (size_t)r.samples * r.width * r.height * r.dims + 16 : 0;
+    trim_sample_rows(ctx, floats);
     if(ctx->sample_rows.count < floats)
     {
         try
@@ -2016,7 +2036,7 @@ SampleRows plan_sample_rows(btrc_ctx *ctx, const btrc_render_params *p, const st
         }
         catch(const std::bad_alloc &)
         {
-            (void)hipGetLastError(); // no room: the digit loop needs none
+            (void)hipGetLastError();
             return SampleRows();
         }
     }
@@ -2064,6 +2084,8 @@ void render(btrc_ctx *ctx, const btrc_render_params *p, int32_t view_count, cons
     // pool sides: the last bounce's stripes, then the generated states;
     // shadow queue: one stripe per COUNTER_STRIPES-th of the inputs
     const size_t PS = pool_capacity(P), SS = shadow_capacity(P);
+    if(ctx->pool_size != P || ctx->film.count < 4 * pixels)
+        trim_sample_rows(ctx, 0);
     if(ctx->pool_size != P)
     {
         ctx->pool[0].alloc(PS);
@@ -2190,7 +2212,7 @@ void render(btrc_ctx *ctx, const btrc_render_params *p, int32_t view_count, cons
         const int32_t tail = ctx->nrc.params.train ? ctx->nrc.params.train_depth : 0;
         bounces = std::min<int64_t>(bounces, (int64_t)std::max(ctx->nrc.params.query_depth, tail) + 1);
     }
-    const SampleRows rows = plan_sample_rows(ctx, p, views, pixels, media, bounces);
+    const SampleRows rows = alloc_sample_rows(ctx, plan_sample_rows(p, views, pixels, media, bounces));
     const int sampler = rows.samples > 0 ? (int)SAMPLER_HALTON_ROWS : (int)p->sampler;
     rc.rows = rows.samples > 0 ? ctx->sample_rows.ptr : nullptr;
     rc.row_dims = rows.dims;

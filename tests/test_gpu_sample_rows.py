@@ -6,7 +6,7 @@ rendered separately, at a sample offset; tile order equals uniform order."""
 import numpy as np
 import pytest
 
-from btrc_amd import scenes
+from btrc_amd import _abi, scenes
 from oracle import oracle
 
 from util import render_params
@@ -72,3 +72,38 @@ def test_tile_order_equals_uniform(ctx):
     b, rb = fp64_film(ctx, 600, 400, 3, tile=1, state_count=100000)
     assert ra == rb
     assert np.abs(a - b).max() <= 1e-12 * max(1.0, np.abs(a).max())
+
+
+def test_rows_give_their_memory_back(ctx):
+    """rows of two gigabytes are released by the next frame that needs none or
+    far fewer and by a new scene, kept by frames that use them, and taken again
+    beside another pool"""
+    import ctypes as C
+    hip = C.CDLL("libamdhip64.so.7")   # the runtime the library itself links
+    free, total = C.c_size_t(), C.c_size_t()
+
+    def used():
+        assert hip.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+        return (total.value - free.value) / 2.0 ** 20
+
+    def large():
+        p = render_params(512, 384, 32, max_depth=2, state_count=1 << 16)
+        ctx.render(p)     # media rows: 16,384 x 1,000 floats a sample
+        return used()
+
+    scene, cam = scenes.cornell_media(grid=scenes.fbm_grid(8, octaves=3, seed=3, max_sigma=0.2))
+    ctx.upload_scene(scene)
+    ctx.set_camera(cam, 512, 384)
+    one = render_params(512, 384, 1, max_depth=2, state_count=1 << 16)
+    independent = render_params(512, 384, 1, max_depth=2, state_count=1 << 16)
+    independent.sampler = _abi.SAMPLER_INDEPENDENT
+    ctx.render(independent)
+    before = used()
+    for change in (lambda: ctx.render(independent), lambda: ctx.render(one), lambda: ctx.upload_scene(scene)):
+        assert large() > before + 1900
+        assert large() > before + 1900
+        change()
+        assert used() < before + 100
+    assert large() > before + 1900
+    ctx.render(render_params(512, 384, 32, max_depth=2, state_count=1 << 17))
+    assert used() > before + 1900
