@@ -18,21 +18,17 @@
 #include "../kernels/bvh_gpu.h"
 #include "../kernels/wavefront.h"
 #include "bvh_build.h"
+#include "noalloc.h"
 
 using namespace btrc;
 
 // Scratch of btrc_hip_trace_closest_noalloc, for callers that cannot
-// allocate: the batch's ray counters in the first NOALLOC_COUNTER_BYTES, then the
-// traversal's per-lane stack entries beyond the LDS part ([entry][lane]). Every GPU the library runs on holds one
-// copy until the process ends. Host code never uses the array's name as an
-// address: it resolves the device address once per device
-// (hipGetSymbolAddress, at context creation) and uses that.
-// 64 MiB holds the entries of 16 wavefronts per CU for a tree that needs 43 (a
-// million triangles); 8 MiB held 2 (1M incoherent rays: 2.27 ms, now 0.44).
-// Trees whose one wavefront needs more than NOALLOC_WAVE_BYTES are refused.
-constexpr size_t NOALLOC_SCRATCH_BYTES = (size_t)64 << 20;
-constexpr size_t NOALLOC_WAVE_BYTES = ((size_t)8 << 20) - 2048;
-constexpr size_t NOALLOC_COUNTER_BYTES = FETCH_WORDS * sizeof(uint32_t);
+// allocate (sizes: noalloc.h). Every GPU the library runs on holds one copy
+// until the process ends. Host code never uses the array's name as an address:
+// it resolves the device address once per device (hipGetSymbolAddress, at
+// context creation) and uses that.
+static_assert(NOALLOC_COUNTER_BYTES == FETCH_WORDS * sizeof(uint32_t), "the counters come first");
+static_assert(TRACE_BLOCK * sizeof(uint2) == 64 * 8, "stack entries as noalloc.h counts them");
 static __device__ __align__(256) unsigned char scratch[NOALLOC_SCRATCH_BYTES];
 
 namespace {
@@ -3241,16 +3237,11 @@ int btrc_hip_trace_closest_noalloc(btrc_ctx *ctx, const btrc_ray *rays, int64_t 
         check_range(rays, (size_t)n * sizeof(btrc_ray), "rays");
         check_range(hits, (size_t)n * sizeof(btrc_hit), "hits");
         // the persistent grid, capped so that its stack entries fit the scratch
-        const size_t deep = ctx->stack_size > SHORT_STACK_MIN ? (size_t)(ctx->stack_size - SHORT_STACK_MIN) : 0;
-        const size_t per_wave = deep * TRACE_BLOCK * sizeof(uint2);
-        const size_t room = NOALLOC_SCRATCH_BYTES - NOALLOC_COUNTER_BYTES;
-        int waves = ctx->trace_grid;
-        if(per_wave > 0 && (size_t)waves * per_wave > room)
-            waves = (int)(room / per_wave);
-        if(per_wave > NOALLOC_WAVE_BYTES || waves < 1)
-            throw InvalidArg("scene tree too deep for the no-allocation scratch: " + std::to_string(ctx->stack_size) +
-                             " stack entries need " + std::to_string(per_wave) + " bytes per wavefront beyond the " +
-                             std::to_string(NOALLOC_WAVE_BYTES) + " the scratch allows");
+        const int waves = noalloc_waves(ctx->stack_size, SHORT_STACK_MIN, ctx->trace_grid);
+        if(waves < 1)
+            throw InvalidArg("scene tree too deep for the no-allocation scratch: it needs " +
+                             std::to_string(ctx->stack_size) + " stack entries, the scratch allows " +
+                             std::to_string(NOALLOC_STACK_MAX));
         uint8_t *base = static_cast<uint8_t *>(ctx->noalloc_scratch);
         uint32_t *fetch = reinterpret_cast<uint32_t *>(base);
         const size_t lanes = (size_t)waves * TRACE_BLOCK;

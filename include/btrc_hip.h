@@ -493,8 +493,8 @@ int btrc_hip_trace_any(btrc_ctx *ctx, const btrc_ray *rays, int64_t n, int32_t t
  * allocations holding n entries each). It allocates nothing: the
  * traversal's ray counter and its per-lane stack entries beyond the LDS part
  * live in a static 64 MiB device array per GPU, which caps the persistent
- * grid and fails with BTRC_ERR_INVALID when the scene's tree needs more
- * stack than the array holds. Calls that overlap on one GPU race, since they
+ * grid. Fails with BTRC_ERR_INVALID when the scene's tree needs more than
+ * 16,396 stack entries. Calls that overlap on one GPU race, since they
  * share that array. Returns once the hits are written. */
 int btrc_hip_trace_closest_noalloc(btrc_ctx *ctx, const btrc_ray *rays, int64_t n, int32_t tri_test, btrc_hit *hits);
 
