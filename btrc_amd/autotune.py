@@ -22,7 +22,7 @@ from . import _abi
 
 WAVES = (16, 20, 24, 28)
 STAGE_BLOCKS = (8, 16, 32)
-GRAPH_BOUNCES = (2, 4, 8)
+GRAPH_BOUNCES = (0, 2, 4, 8)  # 0: the library's choice (four, or a small frame whole)
 # path pools of 2^21 .. 2^25 states (about 1 to 17 GB of device memory;
 # larger pools mean fewer, larger launches per frame)
 POOLS = (1 << 21, 1 << 23, 1 << 25)
@@ -87,7 +87,7 @@ def autotune(ctx, params, spp=4, waves=WAVES, two_level=False, stage_blocks=STAG
     if pools or graph_bounces:
         ctx.set_tuning(launch_graph=1)
         timed = []
-        for pool, g in itertools.product(pools or (params.state_count,), graph_bounces or (4,)):
+        for pool, g in itertools.product(pools or (params.state_count,), graph_bounces or (0,)):
             q.state_count = pool
             ctx.set_tuning(graph_bounces=g)
             s = _staged(ctx, q).seconds
