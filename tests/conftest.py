@@ -18,6 +18,7 @@ def pytest_configure(config):
 def _session_ctx():
     import btrc_amd
     c = btrc_amd.Context(0)
+    c.default_tuning = c.get_tuning()
     yield c
     c.close()
 
@@ -25,11 +26,10 @@ def _session_ctx():
 @pytest.fixture
 def ctx(_session_ctx):
     """one context for the whole session; every test starts from the box
-    filter, the default tuning and the cache switched off"""
+    filter, a fresh context's tuning and the cache switched off"""
     c = _session_ctx
     c.set_filter("box")
-    c.set_tuning(closest_postpone_leaves=0, any_postpone_leaves=0, trace_waves_per_cu=20, launch_graph=1,
-                 two_level_postpone=0, stage_blocks_per_cu=0, graph_bounces=0)
+    c.set_tuning(**c.default_tuning)
     c.nrc_configure(enabled=0, train_depth=0)
     yield c
 

@@ -109,8 +109,11 @@ def test_any_magnitude_equals_brute_force(ctx, accel, scale, length):
     assert np.array_equal(ctx.trace_any(rays), ref.trace(rays, any_hit=True, use_bvh=False))
 
 
-@pytest.mark.parametrize("n", [1, 63, 64, 65, 1000, 24 * 256 * 64 + 1])
+# around a wavefront, and around the rays that are handed out by workgroup index:
+# 20 (visibility) and 24 (closest hit) wavefronts on each of 256 CUs
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 1000] + [w * 256 * 64 + k for w in (20, 24) for k in (-1, 0, 1)])
 def test_batch_sizes(ctx, n):
+    assert ctx.get_tuning()["trace_waves_per_cu"] == 24
     scene = scenes.sphere_field(instances=64, lights=2, seed=9, extent=12.0)[0]
     ctx.upload_scene(scene)
     rays = random_rays(n, 0.0, 12.0, n)
