@@ -1562,15 +1562,17 @@ __global__ void k_halton_eval(HaltonConsts hc, HaltonTables tab, const uint32_t 
     const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if(i >= n)
         return;
-    // even samples as the stages evaluate them (tables, 32-bit indices), odd
-    // ones and indices beyond 32 bits by the digit loop alone
+    // as the stages evaluate them: even samples with the tables, odd ones by
+    // the digit loop alone (a render's indices fit 32 bits); indices beyond
+    // that by the general loop
     HaltonState hs = halton_start(hc, px[i], py[i], si[i]);
-    const bool tabled = !(i & 1) && (hs.index >> 32) == 0;
+    const uint32_t index = (uint32_t)hs.index;
     for(int32_t k = 0; k < dims; ++k)
     {
         const uint32_t dim = halton_wrap(hs.dimension, 1);
-        out[(size_t)i * dims + k] = tabled ? halton_value(tab, dim, (uint32_t)hs.index)
-                                           : sample_halton(c_primes.p, dim, hs.index);
+        out[(size_t)i * dims + k] = (hs.index >> 32) != 0 ? sample_halton(c_primes.p, dim, hs.index)
+                                    : (i & 1)             ? halton_value_digits(tab, dim, index)
+                                                          : halton_value(tab, dim, index);
         hs.dimension = dim + 1;
     }
 }

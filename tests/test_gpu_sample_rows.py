@@ -74,6 +74,29 @@ def test_tile_order_equals_uniform(ctx):
     assert np.abs(a - b).max() <= 1e-12 * max(1.0, np.abs(a).max())
 
 
+def test_draws_past_the_last_dimension(ctx):
+    """paths that draw more numbers than the 998 dimensions of a row start over
+    at the first: a frame that tracks from rows (staged in chunks) equals the
+    same camera as one of two views, where the small one keeps the digit loop"""
+    grid = scenes.fbm_grid(10, octaves=3, seed=5, max_sigma=0.02).copy()
+    grid[0, 0, 0] = 30.0   # 30 steps a unit, 40 units across, few of them real
+    scene, cam = scenes.cornell_media(grid=grid)
+    ctx.upload_scene(scene)
+    w, h = 512, 384
+    p = render_params(w, h, 1, max_depth=3, state_count=1 << 18)
+    ctx.set_camera(cam, w, h)
+    ctx.render(p)
+    rows = ctx.film(w, h)[0]
+    ctx.render_views(p, [(cam, w, h), (cam, 8, 8)])
+    digits = ctx.view_film(0, w, h)
+    np.testing.assert_allclose(rows, digits, rtol=1e-5, atol=1e-6)
+    oracle.tracking_stats()
+    ref = oracle.OracleScene(scene).render(cam, p, first=(h // 2) * w, count=w)[0][h // 2]
+    segments, lookups = oracle.tracking_stats()
+    assert lookups > 998 * segments / 2   # two draws a lookup
+    assert (np.abs(rows[h // 2, :, :3] - ref) / np.maximum(np.abs(ref), 1e-2)).max() <= 1e-4 and ref.max() > 0
+
+
 def test_rows_give_their_memory_back(ctx):
     """rows of two gigabytes are released by the next frame that needs none or
     far fewer and by a new scene, kept by frames that use them, and taken again
