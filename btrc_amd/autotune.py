@@ -22,7 +22,7 @@ from . import _abi
 
 WAVES = (16, 20, 24, 28)
 STAGE_BLOCKS = (8, 16, 32)
-GRAPH_BOUNCES = (0, 2, 4, 8)  # 0: the library's choice (four, or a small frame whole)
+GRAPH_BOUNCES = (0, 2, 4, 8)  # 0: the library's choice (a frame that fits the pool whole, or four)
 # path pools of 2^21 .. 2^25 states (about 1 to 17 GB of device memory;
 # larger pools mean fewer, larger launches per frame)
 POOLS = (1 << 21, 1 << 23, 1 << 25)

@@ -1974,11 +1974,15 @@ std::vector<ViewRec> make_views(btrc_ctx *ctx, const btrc_render_params *p, int3
 // samples and dimensions its rows hold (samples 0: the stages run the digit
 // loop). Rows hold every dimension a path can draw: four for the camera, eight
 // per vertex of at most `bounces` (all 998 with media, whose tracking steps
-// draw without a bound). They pay off once enough pixels share each
-// (ROWS_MIN_SHARE: 640x360, 14 pixels a row, gains 3 %; 256^2 at 16 spp, 4
-// pixels a row, 1,934 us without and 2,082 with them), and for frames so small
-// that the digit loops' latency counts, not their number (ROWS_SMALL_VALUES: a
-// 320x180 preview's 1.2 million values, 566 us without and 514 with them).
+// draw without a bound). They pay off
+// - once enough pixels share each (ROWS_MIN_SHARE): digit loop against rows at
+//   16 spp and depth 8, a room and a field of spheres, 8 pixels a row 0.94 and
+//   0.98, 12 pixels 0.98 and 1.00, 14 pixels 0.99 and 1.00, 20 pixels 1.01 and
+//   1.01, 29 pixels 1.03 and 1.02; with media at 8 spp 1.44 at 12 pixels;
+// - for frames so small that the digit loops' latency counts, not their number
+//   (ROWS_SMALL_VALUES), however few pixels share a row: 1.2 Mi values 1.10
+//   and 1.03, 4.8 Mi 1.02 and 1.00, 10.7 Mi 0.91 and 0.97.
+// (Media gain below both lines too: 128^2 at 1 spp, 15.6 Mi values, 1.56.)
 // Frames of more samples than ROWS_MAX_BYTES holds go through in windows of
 // samples, which needs sample-major paths: one view in uniform order.
 constexpr int64_t ROWS_MIN_SHARE = 12;
@@ -2290,9 +2294,13 @@ void render(btrc_ctx *ctx, const btrc_render_params *p, int32_t view_count, cons
     // ONE_BLOCK_BOUNCES of them (odd numbers too) run as one block with one
     // read-back, generating in the first bounce only, unless somebody follows
     // the progress. A stop request that finds it running takes effect at its
-    // end: the first four bounces hold most of a frame's time. Blocks of four
-    // leave up to three empty bounces and two read-backs more (four two-level
-    // views of 3.9 M paths: 18.02 ms in one block, 18.35 in three).
+    // end, hence the limit: the first four bounces hold most of a frame's time,
+    // but one block stays faster for any number of them. Blocks of four leave
+    // up to three empty bounces and more read-backs: blocks of four against one
+    // block, a room and a field of spheres at 320x180, 4 bounces 1.04 and 1.01,
+    // 5 bounces 1.27 and 1.19, 9 bounces 1.26 and 1.19, 13 bounces 1.25 and
+    // 1.19; at 1280x720, 9 bounces 1.11 and 1.13; four two-level views of 3.9 M
+    // paths 18.35 and 18.02 ms.
     constexpr int ONE_BLOCK_BOUNCES = 10;
     const int64_t most_rays = (int64_t)std::min<uint64_t>((uint64_t)p->state_count, total);
     const bool one_block = use_graph && ctx->tuning.graph_bounces == 0 && !ctx->reporter.progress &&

@@ -10,7 +10,7 @@ import pytest
 from btrc_amd import _abi, scenes
 from oracle import oracle
 
-from util import assert_hits_equal, random_rays
+from util import assert_hits_equal, random_rays, render_params
 
 pytestmark = pytest.mark.gpu
 
@@ -122,15 +122,20 @@ def test_batch_sizes(ctx, n):
     assert np.array_equal(ctx.trace_any(rays), want["instance"] != 0xffffffff)
 
 
-def test_deep_stacks(ctx):
-    # a fan of nested, overlapping slabs: every box holds every ray, so the
-    # stack grows past its LDS part in every lane
+def slab_scene():
+    """a fan of nested, overlapping slabs: every box holds every ray, so the
+    stack grows past its LDS part in every lane"""
     rng = np.random.default_rng(3)
     n = 6000
     c = rng.uniform(-1, 1, (n, 1, 3)) * np.array([40.0, 0.01, 40.0])
     tris = (c + rng.uniform(-1, 1, (n, 3, 3)) * np.array([30.0, 0.5, 30.0])).astype(np.float32).reshape(n, 9)
     s = scenes.Scene()
     s.add_instance(s.add_geometry(tris), s.add_diffuse([0.5, 0.5, 0.5]))
+    return s
+
+
+def test_deep_stacks(ctx):
+    s = slab_scene()
     ctx.upload_scene(s)
     assert ctx.scene_info()["stack"] > 16
     rays = random_rays(3000, [-40, -1, -40], [40, 1, 40], 8)
@@ -138,3 +143,24 @@ def test_deep_stacks(ctx):
     want = oracle.OracleScene(s).trace(rays, use_bvh=False)
     assert_hits_equal(ctx.trace_closest(rays), want)
     assert np.array_equal(ctx.trace_any(rays), want["instance"] != 0xffffffff)
+
+
+@pytest.mark.parametrize("w,h", [(1024, 1024), (250, 131)])  # on two streams, in one launch
+def test_shadow_and_extension_rays_keep_their_deep_stacks_apart(ctx, w, h):
+    """a bounce's shadow rays are traced beside the next bounce's extension
+    rays: with both past the LDS part of their stacks, the frame equals the
+    one whose launches run one by one"""
+    s = slab_scene()
+    s.add_instance(0, 0, scenes.translate(0.0, 4.0, 0.0))   # bounces go on between the two
+    s.set_gradient_sky((0.0, 1.0, 0.0), (0.1, 0.2, 0.3), (0.6, 0.5, 0.4))
+    ctx.upload_scene(s)
+    assert ctx.scene_info()["stack"] > 16
+    ctx.set_camera(scenes.Camera((30.0, 2.0, 0.0), (0.0, 2.0, 5.0), (0.0, 1.0, 0.0), 60.0), w, h)
+    got = []
+    for graph in (1, 0):
+        ctx.set_tuning(launch_graph=graph)
+        st = ctx.render(render_params(w, h, 1, max_depth=6, state_count=1 << 20, film_fp64=1))
+        got.append((st.extension_rays, st.shadow_rays, ctx.film(w, h, fp64=True)[1]))
+    (ea, sa, a), (eb, sb, b) = got
+    assert ea == eb > 1.5 * w * h and sa == sb > 0.3 * w * h
+    assert np.abs(a - b).max() <= 1e-12 * max(1.0, np.abs(b).max())
