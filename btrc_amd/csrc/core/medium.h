@@ -134,7 +134,8 @@ BTRC_HD float grid_lookup(const float *g, int32_t nx, int32_t ny, int32_t nz, in
 // lookup come from one line, where the plain grid's four rows lie in four or
 // five (a step's random lookups ran into the L2's request rate: 14 TB/s of
 // lines; media frame, 1080p at 4 spp: 46.0 ms of tracking, 36.3 from bricks).
-// Four times the grid's memory.
+// Four times the grid's memory (eight for a grid one voxel thin along an axis,
+// sixteen along two).
 constexpr int32_t BRICK_FLOATS = 32;
 
 struct Grids

@@ -173,7 +173,7 @@ struct HitRecord
 // ANY ends a ray at its first hit in [tmin, tmax]. POSTPONE: triangle tests
 // wait until no lane can step through an inner node.
 //
-// Bound by the trips to memory of a node's seven 16-byte loads (VALU busy 66 %
+// Bound by the trips to memory of a node's seven 16-byte loads (VALU busy 69 %
 // of the field frame's launches, 47 % of the lanes active; 80 % and 29 % when
 // each lane tested its whole leaf when it met it: a tenth of the lanes reach
 // a leaf at a time, and a leaf's test takes as long as the wavefront's longest).

@@ -275,8 +275,8 @@ enum : int
     STAGE_COUNT = 7,
 };
 
-// parity: the bounce's parity (the pool side it reads)
-// before the bounce of this parity (first: no bounce came before it)
+// parity, here and below: the bounce's parity (the pool side it reads)
+// the turn to the bounce of this parity (first: no bounce came before it)
 void launch_turn(hipStream_t s, const RenderConsts *rc, WaveCounters *c, int32_t state_count, int parity, bool first);
 // fills the sample rows of `samples` samples from `sample` on, width * height each
 void launch_sample_rows(hipStream_t s, const HaltonConsts &hc, const HaltonTables &tab, int32_t width, int32_t height,
